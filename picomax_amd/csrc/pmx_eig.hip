@@ -1777,6 +1777,183 @@ __global__ void __launch_bounds__(256) bisect_kernel(int N, int nmat, int nb, in
     evals[(size_t)mat * nb + j] = lam;
 }
 
+/* bisect_kernel for batches too small to fill the GPU with one thread per
+ * level: L >= 2 lanes per (matrix, index).  A workgroup takes blockDim / L
+ * consecutive (matrix, index) pairs and stages the d and e^2 of
+ * the mspan matrices these touch in LDS once, so the Sturm passes read LDS
+ * rather than re-streaming T from L2.
+ *
+ * A pass over T at a shift x factors T - xI from both ends towards row
+ * m = N / 2: q_i = d_i - x - e_{i-1}^2 / q_{i-1} down from row 0,
+ * p_i = d_i - x - e_i^2 / p_{i+1} up from row N - 1, and in the middle
+ * g = d_m - x - e_{m-1}^2 / q_{m-1} - e_m^2 / p_{m+1}.  The negative pivots
+ * count the eigenvalues below x (a congruence keeps the inertia) and
+ * s = d/dx log|det(T - xI)| is the sum of q'/q over all pivots, with
+ * q_i' = -1 + e_{i-1}^2 q_{i-1}'/q_{i-1}^2 and the same for p and g.  The two
+ * half chains are independent, which is the point: a pass is a chain of
+ * dependent FP64 operations (about 100 cycles a row), and this halves it.
+ *
+ * Each lane of a group probes its own x.  Until the bracket holds eigenvalue
+ * j alone (count(lo) = j, count(hi) = j + 1) the probes cut it into L + 1
+ * equal parts.  From there lane 0 probes the Newton candidate x - 1/s of the
+ * bracket end that is closer by its own step (the midpoint if that falls
+ * outside), the others cut the bracket into L parts.  It stops when the
+ * bracket or the Newton step is at the rounding level of T: 2 eps |x| + 4
+ * pivmin plus a fraction of eps ||T||, below which counts and steps are noise
+ * (without that term a level near zero never meets the test).  A level takes
+ * about 7 passes with L = 64 and 15 with one thread. */
+template <int L>
+__global__ void __launch_bounds__(256) bisect_group_kernel(int N, int nmat, int nb, int mspan, const double *dS,
+                                                     const double *eS, const double *gb, double *lamS, double *evals) {
+    extern __shared__ double smem_d[];
+    double *dl = smem_d;                      /* [mspan][N] */
+    double *e2l = dl + (size_t)mspan * N;     /* [mspan][N + 1]: e_{i-1}^2 at i, 0 at 0 and N */
+    const size_t g0 = (size_t)blockIdx.x * (blockDim.x / L), gtot = (size_t)nmat * nb;
+    const int m0 = (int)(g0 / nb);
+    const int nm = min(mspan, nmat - m0);
+    for (int idx = threadIdx.x; idx < nm * (N + 1); idx += blockDim.x) {
+        const int i = idx / nm, ml = idx % nm;
+        if (i < N) dl[ml * N + i] = dS[(size_t)i * nmat + m0 + ml];
+        const double e = (i > 0 && i < N) ? eS[(size_t)(i - 1) * nmat + m0 + ml] : 0.0;
+        e2l[ml * (N + 1) + i] = e * e;
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & (L - 1);
+    const size_t g = g0 + threadIdx.x / L;
+    if (g >= gtot) return;
+    const int mat = (int)(g / nb), j = (int)(g % nb);
+    const double *d = dl + (mat - m0) * N, *e2 = e2l + (mat - m0) * (N + 1);
+    double lo = gb[4 * mat], hi = gb[4 * mat + 1];
+    const double pivmin = gb[4 * mat + 2], tnorm = gb[4 * mat + 3];
+    int clo = 0, chi = N; /* counts below lo and hi (the Gershgorin bounds hold every eigenvalue) */
+    double slo = 0.0, shi = 0.0; /* d log|det| at lo and hi; 0 (no step) at the Gershgorin bounds */
+    /* 1/q from v_rcp_f64 and one Newton step (a few ulp; the count is that of
+     * a T perturbed at that level) */
+    auto rcp = [](double q) {
+        double r = __builtin_amdgcn_rcp(q);
+        return fma(fma(-q, r, 1.0), r, r);
+    };
+    const int m = N >> 1, nbot = N - 1 - m; /* rows above and below the middle row; nbot = m or m - 1 */
+    const int wl = threadIdx.x & 63, gbase = wl & ~(L - 1);
+    double x0 = 0.5 * (lo + hi), lam = x0; /* lane 0's probe once the eigenvalue is alone */
+    bool alone = false;
+    for (int it = 0; it < 160; it++) {
+        const double tol = 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + 4.0 * pivmin + 0.0625 * DBL_EPSILON * tnorm;
+        if (hi - lo <= tol) {
+            lam = 0.5 * (lo + hi);
+            break;
+        }
+        /* equally spaced probes lo + u h: u = lane + 1 of L + 1 parts, or (lanes from 1) u = lane of L */
+        const double h = (hi - lo) / (alone ? (double)L : (double)(L + 1));
+        const int u = alone ? lane : lane + 1;
+        const double x = (alone && lane == 0) ? x0 : fma((double)u, h, lo);
+        int cnt = 0;
+        double q = d[0] - x, p = d[N - 1] - x, qp = -1.0, pp = -1.0, rq = 0.0, rp = 0.0, sd = 0.0;
+        if (m > 0) {
+            if (fabs(q) < pivmin) q = -pivmin;
+            cnt += q < 0.0;
+            rq = rcp(q);
+            sd = qp * rq;
+        }
+        if (nbot > 0) {
+            if (fabs(p) < pivmin) p = -pivmin;
+            cnt += p < 0.0;
+            rp = rcp(p);
+            sd = fma(pp, rp, sd);
+        }
+        for (int i = 1; i < nbot; i++) {
+            const double t = e2[i] * rq, tb = e2[N - i] * rp;
+            q = (d[i] - x) - t;
+            p = (d[N - 1 - i] - x) - tb;
+            qp = fma(t * rq, qp, -1.0);
+            pp = fma(tb * rp, pp, -1.0);
+            if (fabs(q) < pivmin) q = -pivmin;
+            if (fabs(p) < pivmin) p = -pivmin;
+            cnt += (q < 0.0) + (p < 0.0);
+            rq = rcp(q);
+            rp = rcp(p);
+            sd = fma(qp, rq, sd);
+            sd = fma(pp, rp, sd);
+        }
+        if (m > 1 && nbot < m) { /* N even: one more row from above */
+            const double t = e2[m - 1] * rq;
+            q = (d[m - 1] - x) - t;
+            qp = fma(t * rq, qp, -1.0);
+            if (fabs(q) < pivmin) q = -pivmin;
+            cnt += q < 0.0;
+            rq = rcp(q);
+            sd = fma(qp, rq, sd);
+        }
+        {
+            const double t = e2[m] * rq, tb = e2[m + 1] * rp;
+            double gm = ((d[m] - x) - t) - tb;
+            const double gp = fma(t * rq, qp, fma(tb * rp, pp, -1.0));
+            if (fabs(gm) < pivmin) gm = -pivmin;
+            cnt += gm < 0.0;
+            sd = fma(gp, rcp(gm), sd);
+        }
+        /* the new bracket: the equally spaced probes below eigenvalue j are the
+         * first k of them, then lane 0's own probe */
+        const bool below = cnt <= j;
+        const unsigned long long bal = (__ballot(below) >> gbase) & (L == 64 ? ~0ull : ((1ull << (L & 63)) - 1));
+        const double olo = lo;
+        const int first = alone ? 1 : 0; /* lanes first..L-1 are the equally spaced ones */
+        const int k = __popcll(bal >> first), np = L - first;
+        const int llo = first + k - 1, lhi = first + k; /* lanes of the new ends (if 0 < k, k < np) */
+        const int sl = gbase + max(llo, 0), sh = gbase + min(lhi, L - 1);
+        const double s_l = __shfl(sd, sl), s_h = __shfl(sd, sh);
+        const int c_l = __shfl(cnt, sl), c_h = __shfl(cnt, sh);
+        if (k > 0) {
+            lo = fma((double)k, h, olo);
+            clo = c_l;
+            slo = s_l;
+        }
+        if (k < np) {
+            hi = fma((double)(k + 1), h, olo);
+            chi = c_h;
+            shi = s_h;
+        }
+        if (alone) {
+            const double s_0 = __shfl(sd, gbase);
+            if (bal & 1) {
+                if (x0 > lo) {
+                    lo = x0;
+                    slo = s_0;
+                }
+            } else if (x0 < hi) {
+                hi = x0;
+                shi = s_0;
+            }
+        }
+        const double mid = 0.5 * (lo + hi);
+        double xn = mid;
+        alone = alone || (clo == j && chi == j + 1);
+        if (alone) {
+            /* eigenvalue j alone in (lo, hi]: Newton on det(T - xI) */
+            const double stl = 1.0 / slo, sth = 1.0 / shi;
+            const bool low = fabs(stl) <= fabs(sth);
+            const double step = low ? stl : sth, xb = low ? lo : hi;
+            const double cand = xb - step;
+            if (fabs(step) <= 2.0 * DBL_EPSILON * fabs(xb) + 4.0 * pivmin + 0.5 * DBL_EPSILON * tnorm && cand >= lo && cand <= hi) {
+                lam = cand;
+                break;
+            }
+            if (cand > lo && cand < hi) xn = cand; /* NaN and inf fail this and bisect */
+        }
+        if (xn == lo || xn == hi) { /* no representable point strictly inside */
+            lam = mid;
+            break;
+        }
+        x0 = xn;
+        lam = mid;
+    }
+    if (j >= N) lam = 0.0;
+    if (lane == 0) {
+        lamS[(size_t)j * nmat + mat] = lam;
+        evals[(size_t)mat * nb + j] = lam;
+    }
+}
+
 /* per matrix, the range [j0, j0 + cnt) of the lowest nvec eigenvalues whose
  * vectors are wanted: vsel 1 keeps lambda > voff (conduction states), vsel 2
  * keeps lambda <= voff (valence states); the eigenvalues are ascending, so
@@ -2814,6 +2991,53 @@ template <class T, int NBP, int NCOL, int TU> int launch_tridiag_panel(pmx_ctx *
     return 0;
 }
 
+/* Lanes per eigenvalue: as many as keep the batch within two waves on every
+ * SIMD, where the Sturm chains' latency stops being hidden by other waves and
+ * more lanes would only add work.  The (matrix, index) pairs of a workgroup
+ * touch at most (256 / L - 1) / nb + 2 matrices; where those do not fit the
+ * LDS (large N) L doubles, and at last one wave per workgroup takes one pair. */
+int launch_bisect(pmx_ctx *c, int N, int nm, int nb, const double *dS, const double *eS, const double *gb,
+                  double *lamS, double *evals) {
+    const size_t pairs = (size_t)nm * nb, fill = (size_t)c->num_cu * 4 * 2 * 64;
+    auto span = [&](int L, int threads) { return threads / L == 1 ? 1 : std::min(nm, (threads / L - 1) / nb + 2); };
+    auto bytes = [&](int L, int threads) { return sizeof(double) * (size_t)span(L, threads) * (2 * (size_t)N + 1); };
+    int L = 1, threads = 256;
+    if (pairs * 2 > fill) { /* one thread per level */
+        int mpw = std::max(1, 256 / nb);
+        while (mpw > 1 && sizeof(double) * 2 * (size_t)mpw * N > c->lds_max) mpw--;
+        const size_t lds_b = sizeof(double) * 2 * (size_t)mpw * N;
+        if (lds_b > c->lds_max) return set_error(PMX_EINVAL, "too many eigenvalues or too large a basis for bisection");
+        if (lds_b > 65536)
+            PMX_CHECK_HIP(hipFuncSetAttribute((const void *)bisect_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (int)lds_b));
+        hipLaunchKernelGGL(bisect_kernel, dim3((nm + mpw - 1) / mpw), dim3(256), lds_b, c->stream, N, nm, nb, mpw, dS,
+                           eS, gb, lamS, evals);
+        PMX_CHECK_HIP(hipGetLastError());
+        return 0;
+    }
+    while (L < 64 && (pairs * L * 2 <= fill || bytes(L, threads) > c->lds_max)) L *= 2;
+    if (bytes(L, threads) > c->lds_max) threads = 64;
+    const size_t lds = bytes(L, threads);
+    if (lds > c->lds_max) return set_error(PMX_EINVAL, "too many eigenvalues or too large a basis for bisection");
+    auto go = [&](auto kern) -> int {
+        const int gpw = threads / L;
+        if (lds > 65536)
+            PMX_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3((unsigned)((pairs + gpw - 1) / gpw)), dim3(threads), lds, c->stream, N, nm, nb,
+                           span(L, threads), dS, eS, gb, lamS, evals);
+        PMX_CHECK_HIP(hipGetLastError());
+        return 0;
+    };
+    switch (L) {
+    case 2: return go(bisect_group_kernel<2>);
+    case 4: return go(bisect_group_kernel<4>);
+    case 8: return go(bisect_group_kernel<8>);
+    case 16: return go(bisect_group_kernel<16>);
+    case 32: return go(bisect_group_kernel<32>);
+    default: return go(bisect_group_kernel<64>);
+    }
+}
+
 /* Autotuner for the tridiagonalisation: several kernels reduce the same
  * matrices to the same tridiagonal form (to rounding), and which is fastest
  * depends on N, the element type and how much of the matrices the caches
@@ -3182,16 +3406,8 @@ static int eig_device_run(pmx_ctx *c, int nmat, const double *dKpts, int nb, int
         }
         {
             Prof pf(c, "bisect", 0.0, 0.0);
-            int mpw = std::max(1, 256 / nb);
-            while (mpw > 1 && sizeof(double) * 2 * (size_t)mpw * N > c->lds_max) mpw--;
-            const size_t lds_b = sizeof(double) * 2 * (size_t)mpw * N;
-            if (nb > 256 || lds_b > c->lds_max) return set_error(PMX_EINVAL, "too many eigenvalues or too large a basis for bisection");
-            if (lds_b > 65536)
-                PMX_CHECK_HIP(hipFuncSetAttribute((const void *)bisect_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                  (int)lds_b));
-            hipLaunchKernelGGL(bisect_kernel, dim3((nm + mpw - 1) / mpw), dim3(256), lds_b, c->stream, N, nm, nb, mpw,
-                               dS, eS, gb, lamS, dEvals + (size_t)m0 * nb);
-            PMX_CHECK_HIP(hipGetLastError());
+            if (nb > 256) return set_error(PMX_EINVAL, "too many eigenvalues or too large a basis for bisection");
+            if ((rc = launch_bisect(c, N, nm, nb, dS, eS, gb, lamS, dEvals + (size_t)m0 * nb))) return rc;
         }
         if (nvec > 0) {
             {

@@ -1,0 +1,58 @@
+"""The eigenvalue kernels that small batches take (several lanes per level) at
+the sizes where they change: held to numpy's eigenvalues of the oracle's H(k),
+1e-10 eV, the bar of the band fixtures."""
+import numpy as np
+import pytest
+
+import orc
+from picomax_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+VG = [3, 4, 8, 11, -0.21, 0, 0.04, 0.08, -0.21, 0, 0.04, 0.08]
+
+
+def _pair(vg, gcut2, neps=1, us=None):
+    gcut = gcut2 ** 0.5
+    args = ["-crystal", "zb", "-a", "5.43", "-vg", ",".join(map(str, vg)), "-gcut", repr(gcut), "-neps", str(neps)]
+    if us:
+        args += ["-us_so", ",".join("%r:%r" % kv for kv in us.items())]
+    inp = capi.Input(args)
+    ctx = capi.Context(0)
+    ctx.set_system(inp.system(), inp)
+    return ctx, orc.System("zb", a=5.43, vg=vg, gcut=gcut, neps=neps, us_so=us)
+
+
+def _eig(s, k):
+    return np.linalg.eigvalsh(s.hamiltonian(k))
+
+
+# nk spans one lane per level to 64, N even and odd, one level and all of them
+@pytest.mark.parametrize("nk", [1, 2, 37, 260, 1500, 9000])
+@pytest.mark.parametrize("gcut2,nband,us", [(12.0, 16, None), (12.0, 1, None), (3.1, 18, None), (0.5, 2, None),
+                                            (4.1, 30, {3: 0.01, 8: 0.005})])
+def test_levels_of_small_batches(nk, gcut2, nband, us):
+    ctx, s = _pair(VG, gcut2, us=us)
+    rng = np.random.default_rng(nk + nband)
+    K = rng.uniform(-0.5, 0.5, (nk, 3))
+    ev = ctx.bands(K, nband)
+    for k in {0, nk // 2, nk - 1}:
+        w = _eig(s, K[k])[:nband]
+        assert np.abs(ev[k, :len(w)] - w).max() < 1e-10, (nk, k)
+    ctx.close()
+
+
+@pytest.mark.parametrize("target", [1e-2, 1e-6, 0.0])
+def test_level_at_zero(target):
+    """A level whose magnitude is far below the rounding level of H."""
+    ctx, s = _pair(VG, 12.0)
+    lo, hi = 0.0, 0.9
+    d = np.array([0.6, 0.64, 0.48])
+    assert _eig(s, lo * d)[0] < 0 < _eig(s, hi * d)[0]
+    for _ in range(60):
+        mid = 0.5 * (lo + hi)
+        lo, hi = (mid, hi) if _eig(s, mid * d)[0] < target else (lo, mid)
+    K = np.array([hi * d] * 5)
+    ev = ctx.bands(K, 8)
+    assert np.abs(ev - _eig(s, K[0])[None, :8]).max() < 1e-10
+    ctx.close()
