@@ -1,15 +1,20 @@
-"""The eigenvalue kernels that small batches take (several lanes per level) at
-the sizes where they change: held to numpy's eigenvalues of the oracle's H(k),
-1e-10 eV, the bar of the band fixtures."""
+"""The eigenvalue kernels that small batches take (several lanes per level),
+and the economised broadening tables, each at the sizes where they change.
+
+Eigenvalues are held to numpy's on the oracle's H(k), 1e-10 eV, the bar of the
+band fixtures.  chi of the binned FP64 path is held to the per-transition sum
+(`direct`) within 1e-8 of each slice's maximum, the bar of the chi fixtures
+(both tables are cut below 1e-11 of the broadening's peak)."""
 import numpy as np
 import pytest
 
 import orc
-from picomax_amd import capi
+from picomax_amd import capi, kpoints
 
 pytestmark = pytest.mark.gpu
 
 VG = [3, 4, 8, 11, -0.21, 0, 0.04, 0.08, -0.21, 0, 0.04, 0.08]
+VG_AB = [3, 4, 8, 11, -0.1407, 0.05, 0.0, 0.0577, -0.2807, -0.05, 0.0, 0.0277]
 
 
 def _pair(vg, gcut2, neps=1, us=None):
@@ -55,4 +60,21 @@ def test_level_at_zero(target):
     K = np.array([hi * d] * 5)
     ev = ctx.bands(K, 8)
     assert np.abs(ev - _eig(s, K[0])[None, :8]).max() < 1e-10
+    ctx.close()
+
+
+# (df/2)/epsilon from nearly 0 to the largest the binned path takes, both broadenings
+@pytest.mark.parametrize("delta,eps,df", [(0, 0.3, 0.02), (0, 0.1, 0.05), (0, 0.1, 0.115), (1, 0.3, 0.02),
+                                          (1, 0.05, 0.02), (1, 0.15, 0.1), (1, 0.1, 0.055)])
+def test_economised_tables(delta, eps, df):
+    ctx, _ = _pair(VG_AB, 8.1, neps=3)
+    K = kpoints.gamma_grid("zb", 3) + np.array([0.013, 0.027, 0.041])
+    KW = np.full(len(K), 1.0 / len(K))
+    off = ctx.ref_energy((0, 0, 0), 8)
+    a = (K, KW, [[0.01, 0.0, 0.0]], 24, off, delta, eps, 120, df, 0)
+    got, want = ctx.chi(*a, precision="fp64"), ctx.chi(*a, precision="direct")
+    for g, w in zip(got, want):
+        g, w = g.reshape(-1, 120), w.reshape(-1, 120)
+        scale = np.maximum(np.abs(w).max(1), 1e-4 * np.abs(w).max())
+        assert (np.abs(g - w).max(1) / scale).max() < 1e-8
     ctx.close()
