@@ -80,6 +80,20 @@ __device__ __forceinline__ zd cdiv(zd a, zd b) {
 __device__ __forceinline__ double cdiv(double a, double b) { return a / b; }
 
 
+/* acc + a b, acc + conj(a) b and acc - a b as chains of FMAs (four for complex) */
+__device__ __forceinline__ double mad(double acc, double a, double b) { return fma(a, b, acc); }
+__device__ __forceinline__ double madc(double acc, double a, double b) { return fma(a, b, acc); }
+__device__ __forceinline__ double msub(double acc, double a, double b) { return fma(-a, b, acc); }
+__device__ __forceinline__ zd mad(zd c, zd a, zd b) {
+    return zd{fma(-a.y, b.y, fma(a.x, b.x, c.x)), fma(a.y, b.x, fma(a.x, b.y, c.y))};
+}
+__device__ __forceinline__ zd madc(zd c, zd a, zd b) {
+    return zd{fma(a.y, b.y, fma(a.x, b.x, c.x)), fma(-a.y, b.x, fma(a.x, b.y, c.y))};
+}
+__device__ __forceinline__ zd msub(zd c, zd a, zd b) {
+    return zd{fma(a.y, b.y, fma(-a.x, b.x, c.x)), fma(-a.y, b.x, fma(-a.x, b.y, c.y))};
+}
+
 /* Sum over a full wave (every lane active) by DPP within rows of 16 and
  * four lane reads; every lane gets the same bits, in every wave alike. */
 template <int CTRL> __device__ __forceinline__ double dpp_f64(double v) {
@@ -102,6 +116,41 @@ __device__ __forceinline__ double wave_sum_full(double v) {
     v += dpp_f64<0x141>(v); /* row_half_mirror */
     v += dpp_f64<0x140>(v); /* row_mirror */
     return (readlane_f64(v, 0) + readlane_f64(v, 16)) + (readlane_f64(v, 32) + readlane_f64(v, 48));
+}
+
+/* Sum of each of eight values over the wave: the lanes of a group of eight
+ * (lane >> 3) end with the total of value wave_sum8_id(lane).  Each exchange
+ * halves the values a lane carries, so eight sums cost 34 instructions where
+ * eight wave_sum_full cost 176. */
+__device__ __forceinline__ double swap_add32(double a, double b) {
+    const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto l = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __longlong_as_double(((unsigned long long)h[0] << 32) | l[0]) +
+           __longlong_as_double(((unsigned long long)h[1] << 32) | l[1]);
+}
+__device__ __forceinline__ double swap_add16(double a, double b) {
+    const unsigned long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto l = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false, false);
+    return __longlong_as_double(((unsigned long long)h[0] << 32) | l[0]) +
+           __longlong_as_double(((unsigned long long)h[1] << 32) | l[1]);
+}
+__device__ __forceinline__ double wave_sum8(const double (&v)[8], int lane) {
+    double s[4], t[2];
+#pragma unroll
+    for (int i = 0; i < 4; i++) s[i] = swap_add32(v[2 * i], v[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i < 2; i++) t[i] = swap_add16(s[2 * i], s[2 * i + 1]);
+    const bool b3 = lane & 8;
+    double r = (b3 ? t[1] : t[0]) + dpp_f64<0x128>(b3 ? t[0] : t[1]); /* row_ror 8: lane ^ 8 of its row */
+    r += dpp_f64<0x141>(r); /* row_half_mirror */
+    r += dpp_f64<0xB1>(r);
+    r += dpp_f64<0x4E>(r);
+    return r;
+}
+__device__ __forceinline__ int wave_sum8_id(int lane) {
+    return ((lane >> 3) & 1) * 4 + ((lane >> 4) & 1) * 2 + (lane >> 5);
 }
 
 /* packed column-major lower storage: element (i, j), i >= j */
@@ -166,6 +215,32 @@ template <> __device__ __forceinline__ zd h_elem<zd>(const EigArgs &a, const dou
     zd isy{-sy.y, sy.x}; /* i * SOy */
     if (si == 1 && sj == 0) return sx + isy;
     return sx - isy; /* (0, 1) */
+}
+
+/* Gershgorin bounds, pivmin and ||T|| of one matrix from d and e in LDS, by
+ * one full wave (minima and maxima: the same bits in any order) */
+__device__ __forceinline__ void write_bounds(const EigArgs &a, int N, int mat, const double *d, const double *e,
+                                             int lane) {
+    double gl = d[0], gu = d[0], emax2 = 0.0;
+    for (int i = lane; i < N; i += 64) {
+        const double off = (i > 0 ? fabs(e[i - 1]) : 0.0) + (i + 1 < N ? fabs(e[i]) : 0.0);
+        gl = fmin(gl, d[i] - off);
+        gu = fmax(gu, d[i] + off);
+        if (i + 1 < N) emax2 = fmax(emax2, e[i] * e[i]);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        gl = fmin(gl, __shfl_xor(gl, o));
+        gu = fmax(gu, __shfl_xor(gu, o));
+        emax2 = fmax(emax2, __shfl_xor(emax2, o));
+    }
+    if (lane == 0) {
+        const double tnorm = fmax(fabs(gl), fabs(gu));
+        a.gb[4 * mat] = gl - (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
+        a.gb[4 * mat + 1] = gu + (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
+        a.gb[4 * mat + 2] = DBL_MIN * fmax(1.0, emax2);
+        a.gb[4 * mat + 3] = tnorm;
+    }
 }
 
 /* deterministic start vector entry in [-1, 1) */
@@ -945,6 +1020,477 @@ __global__ void __launch_bounds__(EIG_THREADS, 2) tridiag_panel_kernel(EigArgs a
             a.gb[4 * mat + 2] = DBL_MIN * fmax(1.0, emax2);
             a.gb[4 * mat + 3] = tnorm;
         }
+        __syncthreads();
+    }
+}
+
+/* tridiag_panel_kernel's scheme for batches that leave CUs idle: one matrix
+ * per CU, eight waves.  With two 256-thread workgroups on a CU and few of
+ * them on the GPU that kernel is bound by the latency of its passes (92 us a
+ * step at N = 582, 61 matrices: 12 GB/s of a CU's 150); here a step has twice
+ * the waves of a workgroup and its passes are arranged for latency:
+ *   - the mat-vec's work item is four neighbouring columns by two blocks of
+ *     64 rows: a wave keeps its partials of those rows in registers over all
+ *     its columns and loads two items (16 loads a lane) ahead, 128 KB in
+ *     flight on the CU;
+ *   - the columns' dot products are reduced four at a time (wave_sum8);
+ *   - W^H v and V^H v are one dot product per wave beside the mat-vec instead
+ *     of 4 j + 1 reductions in the row pass;
+ *   - rows are fixed to threads (row r to thread r mod 512), so a thread reads
+ *     its rows of V and W once per step, before the barrier that precedes
+ *     their use, and the next column and its row of V, W are at hand when the
+ *     step begins.
+ * N = 582, 61 matrices: 53.5 -> 20.4 ms (288 of N = 401: 30.0 -> 20 ms, where
+ * the memory system is the bound: 4.7 TB/s of reads). What is left at N = 582 is
+ * half mat-vec (32k cycles a step of loads, 11k of arithmetic beside them) and
+ * a quarter panel update. */
+constexpr int WD_THREADS = 512, WD_WAVES = 8, WD_NBP = 4, WD_MR = 2;
+
+/* tridiag_wide_kernel's trailing update: rows and columns c0..N-1 of the
+ * packed lower A, panel columns 0..nb-1 of V and W (the rest count as zero).
+ * Per panel column i (complex) one K = 4 step with row entries
+ * (V.x, V.y, W.x, W.y) against column entries (W.x, W.y, V.x, V.y) for the
+ * real part and (-W.y, W.x, -V.y, V.x) for the imaginary; real: two panel
+ * columns per step, (V, W) against (W, V). */
+template <class T>
+__device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int N, int c0, int nb, int lane, int wave) {
+    constexpr bool CX = sizeof(T) == sizeof(zd);
+    constexpr int KS = CX ? WD_NBP : WD_NBP / 2; /* K steps */
+    typedef double dv4 __attribute__((ext_vector_type(4)));
+    const int L = N - c0;
+    if (L <= 0) return;
+    const int nrb = (L + 63) >> 6, ncg = (L + 15) >> 4;
+    asm volatile("" : "+v"(lane)); /* no address hoisted into the caller's loops */
+    const int kq = lane >> 4, lc = lane & 15;
+    struct Item {
+        int rb, cg;
+    };
+    /* items row block by row block: column groups 0 .. min(4 rb + 4, ncg) - 1 */
+    auto settle = [&](Item it) {
+        while (it.rb < nrb && it.cg >= min(4 * it.rb + 4, ncg)) {
+            it.cg -= min(4 * it.rb + 4, ncg);
+            it.rb++;
+        }
+        return it;
+    };
+    /* the panel entry of row or column x that K index kq of step s takes;
+     * swap: V and W exchanged (columns), flip: x and y exchanged (imaginary part) */
+    auto panel = [&](int s, int x, bool swap, bool flip) -> double {
+        const int i = CX ? s : 2 * s + (kq >> 1);
+        const bool w = (CX ? (kq >> 1) : (kq & 1)) != (swap ? 1 : 0);
+        const double *q = reinterpret_cast<const double *>((w ? Wp : Vp) + (size_t)i * N + min(x, N - 1));
+        const double v = CX ? q[(kq & 1) ^ (flip ? 1 : 0)] : q[0];
+        return i < nb ? v : 0.0;
+    };
+    Item it = settle(Item{0, wave});
+    T cur[4][4], nxt[4][4];       /* [row tile][accumulator]: row 16 t + lc, column kq + 4 v */
+    double rf[KS][4];             /* row entries of the current row block */
+    double cr[KS], ci[KS];        /* column entries of the current item */
+    double nr[KS], ni[KS];        /* and of the next */
+    auto load = [&](Item q, T (&b)[4][4], double (&er)[KS], double (&ei)[KS]) {
+        if (q.rb >= nrb) q = Item{0, 0}; /* past the last item: loaded and not used */
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            er[s] = panel(s, c0 + 16 * q.cg + lc, true, false);
+            ei[s] = CX ? panel(s, c0 + 16 * q.cg + lc, true, true) : 0.0;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int c = min(c0 + 16 * q.cg + kq + 4 * v, N - 1);
+            const T *col = A + ((long)pk(c, c, N) - c);
+#pragma unroll
+            for (int t = 0; t < 4; t++) b[t][v] = col[max(min(c0 + 64 * q.rb + 16 * t + lc, N - 1), c)];
+        }
+    };
+    load(it, cur, cr, ci);
+    int have = -1; /* row block in rf */
+    while (it.rb < nrb) {
+        const int r0 = c0 + 64 * it.rb, cc = c0 + 16 * it.cg;
+        if (have != it.rb) {
+            have = it.rb;
+#pragma unroll
+            for (int s = 0; s < KS; s++)
+#pragma unroll
+                for (int t = 0; t < 4; t++) rf[s][t] = panel(s, r0 + 16 * t + lc, false, false);
+        }
+        const Item nx = settle(Item{it.rb, it.cg + WD_WAVES});
+        load(nx, nxt, nr, ni);
+#pragma unroll
+        for (int s = 0; s < KS; s++) { /* the update subtracts; the odd imaginary steps carry their own sign */
+            cr[s] = -cr[s];
+            ci[s] = (kq & 1) ? -ci[s] : ci[s];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            dv4 xr, xi;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                xr[v] = re(cur[t][v]);
+                xi[v] = im(cur[t][v]);
+            }
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                xr = __builtin_amdgcn_mfma_f64_16x16x4f64(cr[s], rf[s][t], xr, 0, 0, 0);
+                if (CX) xi = __builtin_amdgcn_mfma_f64_16x16x4f64(ci[s], rf[s][t], xi, 0, 0, 0);
+            }
+            const int r = r0 + 16 * t + lc;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int c = cc + kq + 4 * v;
+                if (c < N && r >= c && r < N) A[pk(r, c, N)] = mk<T>(xr[v], CX ? xi[v] : 0.0);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) cur[t][v] = nxt[t][v];
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+            cr[s] = nr[s];
+            ci[s] = ni[s];
+        }
+        it = nx;
+    }
+}
+
+template <class T>
+__global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) {
+    extern __shared__ double smem_d[];
+    constexpr int NBP = WD_NBP;
+    const int N = a.N;
+    const int tid0 = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid0 >> 6);
+    int tid = tid0, lane = tid0 & 63;
+    const size_t P = (size_t)N * (N + 1) / 2;
+
+    /* LDS: [v N][dot N][part 8 N] (T) [d N][e N] (double) */
+    char *sp = reinterpret_cast<char *>(smem_d);
+    T *vv = reinterpret_cast<T *>(sp); sp += sizeof(T) * N;
+    T *dotv = reinterpret_cast<T *>(sp); sp += sizeof(T) * N;
+    T *part = reinterpret_cast<T *>(sp); sp += sizeof(T) * N * WD_WAVES;
+    double *d = reinterpret_cast<double *>(sp); sp += sizeof(double) * N;
+    double *e = reinterpret_cast<double *>(sp);
+    __shared__ double sh_alpha[2], red[2 * WD_WAVES];
+    __shared__ T sh_tau;
+    __shared__ T sh_cw[NBP], sh_cv[NBP];   /* conj of row k of W and V */
+    __shared__ T sh_cWv[NBP], sh_cVv[NBP]; /* W^H v, V^H v */
+
+    char *slab = a.scratch + (size_t)blockIdx.x * a.slab;
+    T *A = reinterpret_cast<T *>(slab);
+    T *Vp = reinterpret_cast<T *>(slab + ((P * sizeof(T) + 255) / 256) * 256);
+    T *Wp = Vp + (size_t)NBP * N;
+
+    for (int mat = blockIdx.x; mat < a.nmat; mat += gridDim.x) {
+        const double Kv[3] = {a.K[3 * mat], a.K[3 * mat + 1], a.K[3 * mat + 2]};
+        T *vref = a.vref ? reinterpret_cast<T *>(a.vref) + (size_t)mat * P : nullptr;
+        T *tau_out = a.tauv ? reinterpret_cast<T *>(a.tauv) + (size_t)mat * N : nullptr;
+        for (int c = wave; c < N; c += WD_WAVES)
+            for (int r = c + lane; r < N; r += 64) A[pk(r, c, N)] = h_elem<T>(a, Kv, r, c);
+        __syncthreads();
+
+        for (int k0 = 0; k0 + 1 < N; k0 += NBP) {
+            const int nb = min(NBP, N - 1 - k0);
+            /* this thread's rows: of the next column, and of V and W (columns below j) */
+            T xa[WD_MR], vi[WD_MR][NBP], wi[WD_MR][NBP];
+#pragma unroll
+            for (int m = 0; m < WD_MR; m++) {
+                const int r = tid + WD_THREADS * m;
+                xa[m] = (r >= k0 && r < N) ? A[pk(r, k0, N)] : zero<T>();
+#pragma unroll
+                for (int i = 0; i < NBP; i++) vi[m][i] = wi[m][i] = zero<T>();
+            }
+            for (int j = 0; j < nb; j++) {
+                const int k = k0 + j, L = N - k - 1;
+                /* addresses are formed anew in every step: hoisted out of the loop
+                 * they would spill, and a reload inside the mat-vec would wait for
+                 * its loads ahead */
+                asm volatile("" : "+v"(tid), "+v"(lane));
+                /* (a) column k up to date */
+                T xs[WD_MR];
+                double s = 0.0;
+#pragma unroll
+                for (int m = 0; m < WD_MR; m++) {
+                    const int r = tid + WD_THREADS * m;
+                    T x = xa[m];
+#pragma unroll
+                    for (int i = 0; i < NBP; i++)
+                        if (i < j) x = msub(msub(x, vi[m][i], sh_cw[i]), wi[m][i], sh_cv[i]);
+                    if (r < N) {
+                        if (r == k) d[k] = re(x);
+                        if (r == k + 1) {
+                            sh_alpha[0] = re(x);
+                            sh_alpha[1] = im(x);
+                        }
+                        if (r >= k + 2) s += nrm2(x);
+                    }
+                    xs[m] = x;
+                }
+                s = wave_sum_full(s);
+                if (lane == 0) red[wave] = s;
+                __syncthreads(); /* (1) */
+                /* (b) every thread forms the reflector's scalars from the same sums */
+                double xn2 = 0.0;
+#pragma unroll
+                for (int w = 0; w < WD_WAVES; w++) xn2 += red[w];
+                const T alpha = mk<T>(sh_alpha[0], sh_alpha[1]);
+                double beta;
+                T tau, scal;
+                if (xn2 == 0.0 && im(alpha) == 0.0) {
+                    beta = re(alpha);
+                    tau = zero<T>();
+                    scal = zero<T>();
+                } else {
+                    beta = -copysign(sqrt(nrm2(alpha) + xn2), re(alpha));
+                    tau = cdiv(from_real<T>(beta) - alpha, from_real<T>(beta));
+                    scal = cdiv(from_real<T>(1.0), alpha - from_real<T>(beta));
+                }
+                const bool active = !(re(tau) == 0.0 && im(tau) == 0.0);
+#pragma unroll
+                for (int m = 0; m < WD_MR; m++) {
+                    const int r = tid + WD_THREADS * m;
+                    T v = zero<T>();
+                    if (active && r >= k + 1 && r < N) v = (r == k + 1) ? from_real<T>(1.0) : xs[m] * scal;
+                    if (r >= k + 1 && r < N) {
+                        vv[r] = v;
+                        Vp[(size_t)j * N + r] = v;
+                        if (vref && r >= k + 2) vref[pk(r, k, N)] = v;
+                    }
+                }
+                if (tid == 0) {
+                    e[k] = beta;
+                    sh_tau = tau;
+                    if (tau_out) tau_out[k] = tau;
+                }
+                __syncthreads(); /* (2) */
+                /* (c) stale A22 v, every stored element read once.  Local
+                 * column ct and row rr are k + 1 + ct, k + 1 + rr.  A work item
+                 * is four neighbouring columns (quad qd) by two blocks of 64
+                 * rows (group g); a wave takes the quads wave + 8 i that reach
+                 * the group, group by group, and loads two items ahead. */
+                {
+                    const T *vk1 = vv + k + 1;
+                    const int nquad = (L + 3) >> 2, ngrp = (L + 127) >> 7;
+                    int g = wave < nquad ? 0 : ngrp, qd = wave; /* fewer quads than waves: none */
+                    int gl = g, ql = qd;                        /* the item to load next */
+                    auto step = [&](int &g, int &qd) {
+                        qd += WD_WAVES;
+                        if (qd >= min(nquad, 32 * (g + 1))) {
+                            g++;
+                            qd = wave;
+                        }
+                    };
+                    /* every item issues the same eight loads, so the wait before
+                     * an item counts only its own.  Rows past the end read row
+                     * L - 1 (their v is 0 and their partials are not stored),
+                     * rows above the quad read its first row (masked below),
+                     * columns past the end read the last one (v 0, dot not
+                     * stored); past the last item row 0 of column 0 is loaded
+                     * and not used. */
+                    auto load = [&](T (&b)[2][4]) {
+                        const int q0 = gl < ngrp ? 4 * ql : 0, c0 = k + 1 + q0, nc = L - q0;
+                        const int rb = gl < ngrp ? 128 * gl : -128;
+                        const unsigned base = pk(c0, c0, N) - q0;
+                        const unsigned d1 = nc > 1 ? N - 1 - c0 : 0, d2 = nc > 2 ? d1 + N - 2 - c0 : d1,
+                                       d3 = nc > 3 ? d2 + N - 3 - c0 : d2;
+                        const unsigned off[4] = {base, base + d1, base + d2, base + d3};
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const unsigned r = max(min(rb + 64 * h + lane, L - 1), q0);
+#pragma unroll
+                            for (int t = 0; t < 4; t++)
+                                b[h][t] = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(A) +
+                                                                       (unsigned)sizeof(T) * (r + off[t]));
+                        }
+                        if (gl < ngrp) step(gl, ql);
+                    };
+                    T pt[2], vr[2];
+                    auto open_group = [&]() {
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const int rr = 128 * g + 64 * h + lane;
+                            pt[h] = zero<T>();
+                            vr[h] = rr < L ? vk1[min(rr, L - 1)] : zero<T>();
+                        }
+                    };
+                    auto compute = [&](const T (&b)[2][4]) {
+                        const int q0 = 4 * qd;
+                        T dot[4], vc[4];
+#pragma unroll
+                        for (int t = 0; t < 4; t++) {
+                            dot[t] = zero<T>();
+                            vc[t] = vk1[min(q0 + t, L - 1)];
+                        }
+                        if (q0 + 3 >= L) /* columns past the end */
+#pragma unroll
+                            for (int t = 1; t < 4; t++)
+                                if (q0 + t >= L) vc[t] = zero<T>();
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const int rb = 128 * g + 64 * h;
+                            if (rb > q0) { /* below the diagonal (quads do not straddle blocks) */
+#pragma unroll
+                                for (int t = 0; t < 4; t++) {
+                                    dot[t] = madc(dot[t], b[h][t], vr[h]);
+                                    pt[h] = mad(pt[h], b[h][t], vc[t]);
+                                }
+                            } else if (rb + 63 >= q0) { /* on it; else above it */
+                                const int rr = rb + lane;
+#pragma unroll
+                                for (int t = 0; t < 4; t++) {
+                                    const T av = rr >= q0 + t ? b[h][t] : zero<T>();
+                                    dot[t] = madc(dot[t], av, vr[h]); /* the diagonal is real */
+                                    pt[h] = mad(pt[h], rr == q0 + t ? zero<T>() : av, vc[t]);
+                                }
+                            }
+                        }
+                        const double v8[8] = {re(dot[0]), im(dot[0]), re(dot[1]), im(dot[1]),
+                                              re(dot[2]), im(dot[2]), re(dot[3]), im(dot[3])};
+                        const double tot = wave_sum8(v8, lane);
+                        const int wid = wave_sum8_id(lane), ct = q0 + (wid >> 1);
+                        if ((lane & 7) == 0 && ct < L && (sizeof(T) == sizeof(zd) || !(wid & 1))) {
+                            double *o = reinterpret_cast<double *>(dotv + ct) + (wid & 1);
+                            *o = (q0 >> 7) == g ? tot : *o + tot; /* the column's first group sets it */
+                        }
+                    };
+                    T b0[2][4], b1[2][4], b2[2][4];
+                    load(b0);
+                    load(b1);
+                    open_group();
+                    /* one item: load the second after it, compute it; false at the end */
+                    auto turn = [&](const T (&cur)[2][4], T (&fetch)[2][4]) {
+                        load(fetch);
+                        compute(cur);
+                        const int g0 = g;
+                        step(g, qd);
+                        if (g != g0) {
+#pragma unroll
+                            for (int h = 0; h < 2; h++) {
+                                const int rr = 128 * g0 + 64 * h + lane;
+                                if (rr < L) part[wave * N + rr] = pt[h];
+                            }
+                            open_group();
+                        }
+                        return g < ngrp;
+                    };
+                    if (g < ngrp)
+                        while (turn(b0, b2) && turn(b1, b0) && turn(b2, b1)) {
+                        }
+                    else /* this wave has no part of the product */
+                        for (int rr = lane; rr < L; rr += 64) part[wave * N + rr] = zero<T>();
+                    /* W^H v and V^H v: wave i takes column i of the panel */
+                    if (wave < j) {
+                        T tw = zero<T>(), tv = zero<T>();
+                        for (int rr = lane; rr < L; rr += 64) {
+                            const T w = Wp[(size_t)wave * N + k + 1 + rr], v = Vp[(size_t)wave * N + k + 1 + rr];
+                            tw = madc(tw, w, vk1[rr]);
+                            tv = madc(tv, v, vk1[rr]);
+                        }
+                        const double v8[8] = {re(tw), im(tw), re(tv), im(tv), 0.0, 0.0, 0.0, 0.0};
+                        const double tot = wave_sum8(v8, lane);
+                        const int wid = wave_sum8_id(lane);
+                        if ((lane & 7) == 0 && wid < 4) {
+                            T *o = wid < 2 ? &sh_cWv[wave] : &sh_cVv[wave];
+                            if (sizeof(T) == sizeof(zd) || !(wid & 1)) reinterpret_cast<double *>(o)[wid & 1] = tot;
+                        }
+                    }
+                }
+                /* this thread's rows of V and W, for p and for the next column */
+#pragma unroll
+                for (int m = 0; m < WD_MR; m++) {
+                    const int r = tid + WD_THREADS * m;
+#pragma unroll
+                    for (int i = 0; i < NBP; i++) {
+                        const bool in = i < j && r >= k + 1 && r < N;
+                        vi[m][i] = in ? Vp[(size_t)i * N + r] : zero<T>();
+                        wi[m][i] = in ? Wp[(size_t)i * N + r] : zero<T>();
+                    }
+                }
+                __syncthreads(); /* (3) */
+                /* p with the panel's corrections; w = p - (tau/2)(p^H v) v */
+                T ps[WD_MR], vs[WD_MR];
+                double pr = 0.0, pim = 0.0;
+#pragma unroll
+                for (int m = 0; m < WD_MR; m++) {
+                    const int r = tid + WD_THREADS * m;
+                    T p = zero<T>();
+                    vs[m] = zero<T>();
+                    if (r >= k + 1 && r < N) {
+                        const int rr = r - k - 1;
+                        p = dotv[rr];
+                        vs[m] = vv[r];
+#pragma unroll
+                        for (int w = 0; w < WD_WAVES; w++) p += part[w * N + rr];
+#pragma unroll
+                        for (int i = 0; i < NBP; i++)
+                            if (i < j) p = msub(msub(p, vi[m][i], sh_cWv[i]), wi[m][i], sh_cVv[i]);
+                        p = sh_tau * p;
+                        const T cvp = cj(p) * vs[m];
+                        pr += re(cvp);
+                        pim += im(cvp);
+                    }
+                    ps[m] = p;
+                }
+                pr = wave_sum_full(pr);
+                pim = wave_sum_full(pim);
+                if (lane == 0) {
+                    red[wave] = pr;
+                    red[WD_WAVES + wave] = pim;
+                }
+                /* the next column of the panel */
+#pragma unroll
+                for (int m = 0; m < WD_MR; m++) {
+                    const int r = tid + WD_THREADS * m;
+                    xa[m] = (j + 1 < nb && r >= k + 1 && r < N) ? A[pk(r, k + 1, N)] : zero<T>();
+                }
+                __syncthreads(); /* (4) */
+                double sr = 0.0, si = 0.0;
+#pragma unroll
+                for (int w = 0; w < WD_WAVES; w++) {
+                    sr += red[w];
+                    si += red[WD_WAVES + w];
+                }
+                const T al = (-0.5) * (sh_tau * mk<T>(sr, si));
+#pragma unroll
+                for (int m = 0; m < WD_MR; m++) {
+                    const int r = tid + WD_THREADS * m;
+                    if (r >= k + 1 && r < N) {
+                        const T w = ps[m] + al * vs[m];
+                        Wp[(size_t)j * N + r] = w;
+#pragma unroll
+                        for (int i = 0; i < NBP; i++)
+                            if (i == j) {
+                                vi[m][i] = vs[m];
+                                wi[m][i] = w;
+                            }
+                        if (r == k + 1)
+#pragma unroll
+                            for (int i = 0; i < NBP; i++) {
+                                sh_cw[i] = cj(wi[m][i]);
+                                sh_cv[i] = cj(vi[m][i]);
+                            }
+                    }
+                }
+                __syncthreads(); /* (5) W, row k + 1 of V and W visible; red, part free */
+            }
+            /* the panel's update A22 -= V W^H + W V^H on FP64 MFMA (16x16x4): the
+             * matrix instruction's columns are 16 rows of A22 and its rows 16
+             * columns, so a lane's four accumulators are one row's entries in
+             * four columns and each load covers 256 contiguous bytes.  A work
+             * item is 64 rows by 16 columns, the next one's entries loaded
+             * ahead; V and W come straight from the slab. */
+            wide_update<T>(A, Vp, Wp, N, k0 + nb, nb, lane, wave);
+            __syncthreads();
+        }
+        if (tid == 0) {
+            d[N - 1] = re(A[pk(N - 1, N - 1, N)]);
+            e[N - 1] = 0.0;
+            if (tau_out) tau_out[N - 1] = zero<T>();
+        }
+        __syncthreads();
+        for (int i = tid; i < N; i += WD_THREADS) {
+            a.dS[(size_t)i * a.nmat + mat] = d[i];
+            a.eS[(size_t)i * a.nmat + mat] = e[i];
+        }
+        if (wave == 0) write_bounds(a, N, mat, d, e, lane);
         __syncthreads();
     }
 }
@@ -2991,6 +3537,22 @@ template <class T, int NBP, int NCOL, int TU> int launch_tridiag_panel(pmx_ctx *
     return 0;
 }
 
+size_t lds_wide_bytes(int N, size_t elem) {
+    return elem * (2 + WD_WAVES) * (size_t)N + sizeof(double) * 2 * (size_t)N;
+}
+
+/* one matrix per CU (bases whose vectors and partials fit the LDS) */
+template <class T> int launch_tridiag_wide(pmx_ctx *c, EigArgs &a, int grid, size_t lds) {
+    auto go = [&](auto kern) -> int {
+        if (lds > 65536)
+            PMX_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(WD_THREADS), lds, c->stream, a);
+        PMX_CHECK_HIP(hipGetLastError());
+        return 0;
+    };
+    return go(tridiag_wide_kernel<T>);
+}
+
 /* Lanes per eigenvalue: as many as keep the batch within two waves on every
  * SIMD, where the Sturm chains' latency stops being hidden by other waves and
  * more lanes would only add work.  The (matrix, index) pairs of a workgroup
@@ -3158,6 +3720,23 @@ int tridiag_generic(pmx_ctx *c, EigArgs &a, bool real, bool lds_matrix, int grid
         add_panel("panel8", 8, launch_tridiag_panel<double, 8, 2, 8>, launch_tridiag_panel<zd, 8, 2, 8>);
         add_panel("panel4", 4, launch_tridiag_panel<double, 4, 2, 8>, launch_tridiag_panel<zd, 4, 2, 8>);
         cands.insert(cands.end(), unblocked.begin(), unblocked.end());
+        const size_t ldsw = lds_wide_bytes(N, elem) + 512; /* and its fixed arrays */
+        if (ldsw <= c->lds_max && N <= WD_THREADS * WD_MR && a.slab >= mat_bytes + panel_slab_bytes(N, elem, WD_NBP)) {
+            TuneCand wide{"wide8", [=](int nm) {
+                              EigArgs aa = a;
+                              aa.nmat = nm;
+                              const int g = std::min(std::min(grid, nm), c->num_cu);
+                              return real ? launch_tridiag_wide<double>(c, aa, g, lds_wide_bytes(N, elem))
+                                          : launch_tridiag_wide<zd>(c, aa, g, lds_wide_bytes(N, elem));
+                          }};
+            /* batches below the autotuner's two matrices per CU: one per CU */
+            const char *form = std::getenv("PMX_FORCE_KERNEL");
+            const bool forced = form && std::any_of(cands.begin(), cands.end(), [&](const TuneCand &cd) {
+                                    return std::strcmp(form, cd.name) == 0;
+                                });
+            if (a.nmat < 2 * c->num_cu && !forced) return wide.run(a.nmat);
+            cands.push_back(wide);
+        }
     }
     /* complex bases whose lower triangle fits one workgroup's registers
      * (N <= 132): the register-tiled kernel with 6x6 complex tiles */

@@ -78,3 +78,39 @@ def test_economised_tables(delta, eps, df):
         scale = np.maximum(np.abs(w).max(1), 1e-4 * np.abs(w).max())
         assert (np.abs(g - w).max(1) / scale).max() < 1e-8
     ctx.close()
+
+
+TE = ["-crystal", "te", "-a", "4.45", "-f", "1.33", "-u", "0.26", "-vg",
+      "0.565323,1.333333,1.898656,2.261292,3.594626,4.0" + ",-0.2105,-0.1322,0.0451,0.0214,0.0127,-0.0093" * 3]
+TE_SO = ["-us_so", "0.565323:0.0152,1.333333:-0.0061,1.898656:0.0083",
+         "-ua_so", "0.565323:0.0117,1.333333:0.0042,1.898656:-0.0071"]
+SI = ["-crystal", "zb", "-a", "5.43", "-vg", ",".join(map(str, VG))]
+
+
+# bases whose matrix lies in global memory: the smallest, sizes around multiples
+# of 64 and 128 rows, complex, spinor and real, one matrix to more than one per CU
+@pytest.mark.parametrize("args,gcut2,nk", [(TE, 9.0, 1), (TE, 9.6, 3), (TE, 16.0, 300), (TE + TE_SO, 5.0, 2),
+                                           (TE + TE_SO, 9.0, 5), (TE + TE_SO, 16.0, 2), (TE + TE_SO, 20.0, 2),
+                                           (SI, 36.0, 2), (SI, 48.0, 3)])
+def test_vectors_of_large_bases(args, gcut2, nk):
+    """Eigenvalues against numpy (1e-10 eV) and residuals of the pairs (1e-12 of ||H||): what the
+    tridiagonalisation and its reflectors decide."""
+    inp = capi.Input(args + ["-gcut", repr(gcut2 ** 0.5)])
+    ctx = capi.Context(0)
+    ctx.set_system(inp.system(), inp)
+    d = dict(zip(args[::2], args[1::2]))
+    maps = [{float(k): float(v) for k, v in (p.split(":") for p in d[o].split(","))} if o in d else None
+            for o in ("-us_so", "-ua_so")]
+    s = orc.System(d["-crystal"], a=float(d["-a"]), f=float(d["-f"]) if "-f" in d else None,
+                   u=float(d["-u"]) if "-u" in d else None, vg=[float(x) for x in d["-vg"].split(",")],
+                   gcut=gcut2 ** 0.5, us_so=maps[0], ua_so=maps[1])
+    rng = np.random.default_rng(nk)
+    K = rng.uniform(-0.4, 0.4, (nk, 3))
+    ev, vec = ctx.eig(K, 24, vectors=True)
+    for k in {0, nk - 1}:
+        H = s.hamiltonian(K[k])
+        w = np.linalg.eigvalsh(H)
+        z = vec[k].T
+        assert np.abs(ev[k] - w[:24]).max() < 1e-10
+        assert np.abs(H @ z - z * ev[k]).max() < 1e-12 * np.abs(w).max()
+    ctx.close()
