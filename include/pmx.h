@@ -212,8 +212,8 @@ int pmx_epsinv(pmx_ctx *ctx, int nq, int neps, int nfreq, const double *ReX, con
  * device arrays whose leading [nq][neps(neps+1)/2][nfreq] doubles are the
  * i = j = 0 block (pmx_chi_device's output qualifies); dEpsM [nq][nfreq]
  * complex and dElf [nq][nfreq] are device outputs, as pmx_epsinv's epsM /
- * elf.  The Gauss-Jordan workspace is a fixed 32 MiB device array per GPU,
- * set up by pmx_create; neps above 1024 (more than 32 MiB for one matrix) is
+ * elf.  The elimination workspace is a fixed 32 MiB device array per GPU,
+ * set up by pmx_create (used for neps above 127); neps above 1024 is
  * rejected with PMX_EINVAL.  All calls on one GPU share that workspace:
  * calls that overlap on one GPU (several host threads, several contexts)
  * race.  Synchronous on the context's stream. */

@@ -2258,30 +2258,16 @@ __global__ void place_kernel(int nel, int nfreq, int ne2, int nq, int q, const d
     }
 }
 
-/* eps_mn = delta_mn + chi_mn of one diagonal block [q][m][n <= m][f] (n <= m
- * stored, eps_nm = conj(eps_mn)), Gauss-Jordan with partial pivoting on
- * [eps | I], one block per (q, f); epsM = 1/[eps^-1]_00, ELF = -Im [eps^-1]_00
- * (macroscopic.m:23-38, 87-89).  With qg2 ([nq][N], eV^2) the diagonal gets
- * -qg2[q][m] / w_f^2, w_f = f dfreq (macroscopic.m:70-78); f = 0 then gives NaN.
- * head ([nq][nfreq] complex, or null) replaces element (0, 0) (macroscopic.m:18-20). */
-__global__ void __launch_bounds__(256) epsinv_kernel(int N, int nq, int nfreq, const double *ReX, const double *ImX,
-                                                     const double *qg2, double dfreq, const zd *head, zd *work,
-                                                     zd *epsM, double *elf, zd *inv_out, int mat0) {
-    const int mat = mat0 + blockIdx.x; /* matrix (q, f); workspace slot blockIdx.x */
+/* eps_mn = delta_mn + chi_mn of the i = j = 0 block [q][m][n <= m][f] (n <= m
+ * stored, eps_nm = conj(eps_mn)) and its whole inverse: Gauss-Jordan with
+ * partial pivoting on [eps | I], one block per (q, f); epsM = 1/[eps^-1]_00,
+ * ELF = -Im [eps^-1]_00 (macroscopic.m:23-38, 87-89). */
+__global__ void __launch_bounds__(256) epsinv_kernel(int N, int nfreq, const double *ReX, const double *ImX, zd *work,
+                                                     zd *epsM, double *elf, zd *inv_out) {
+    const int mat = blockIdx.x; /* matrix (q, f) and workspace slot */
     const int q = mat / nfreq, f = mat % nfreq;
     const int ne2 = N * (N + 1) / 2;
     const int W = 2 * N;
-    if (qg2 && f == 0) {
-        /* w = 0: an infinite diagonal, no finite inverse */
-        if (threadIdx.x == 0) {
-            epsM[(size_t)q * nfreq + f] = zd{NAN, NAN};
-            elf[(size_t)q * nfreq + f] = NAN;
-        }
-        if (inv_out)
-            for (int e = threadIdx.x; e < N * N; e += blockDim.x) inv_out[(size_t)mat * N * N + e] = zd{NAN, NAN};
-        return;
-    }
-    const double iw2 = qg2 ? 1.0 / ((dfreq * f) * (dfreq * f)) : 0.0;
     zd *A = work + (size_t)blockIdx.x * N * W;
     __shared__ int piv;
     __shared__ double best[256];
@@ -2295,9 +2281,7 @@ __global__ void __launch_bounds__(256) epsinv_kernel(int N, int nq, int nfreq, c
             if (n > m) { int t = m; m = n; n = t; cj = true; }
             const size_t src = ((size_t)q * ne2 + (size_t)m * (m + 1) / 2 + n) * nfreq + f;
             v = zd{ReX[src], cj ? -ImX[src] : ImX[src]};
-            if (head && r == 0 && cidx == 0) v = head[(size_t)q * nfreq + f];
-            else if (r == cidx) v.x += 1.0;
-            if (qg2 && r == cidx) v.x -= qg2[(size_t)q * N + r] * iw2;
+            if (r == cidx) v.x += 1.0;
         } else if (cidx - N == r) {
             v = zd{1.0, 0.0};
         }
@@ -2358,11 +2342,311 @@ __global__ void __launch_bounds__(256) epsinv_kernel(int N, int nq, int nfreq, c
         epsM[(size_t)q * nfreq + f] = zd{g.x / den, -g.y / den};
         elf[(size_t)q * nfreq + f] = -g.y;
     }
-    if (inv_out)
-        for (int e = threadIdx.x; e < N * N; e += blockDim.x) {
-            const int r = e / N, cidx = e % N;
-            inv_out[((size_t)mat * N + r) * N + cidx] = A[(size_t)r * W + N + cidx];
+    for (int e = threadIdx.x; e < N * N; e += blockDim.x) {
+        const int r = e / N, cidx = e % N;
+        inv_out[((size_t)mat * N + r) * N + cidx] = A[(size_t)r * W + N + cidx];
+    }
+}
+
+/* epsM and ELF alone (no inverse) of one diagonal block of chi, as above: with
+ * qg2 ([nq][N], eV^2) the diagonal gets -qg2[q][m] / w_f^2, w_f = f dfreq
+ * (macroscopic.m:70-78); f = 0 then gives NaN.  head ([nq][nfreq] complex, or
+ * null) replaces element (0, 0) (macroscopic.m:18-20). */
+
+/* maximum over the wave, every lane active; every lane gets it */
+template <int CTRL> __device__ __forceinline__ double max_dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_mov_dpp((int)(b & 0xffffffff), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
+    return fmax(v, __longlong_as_double(((long long)hi << 32) | (unsigned)lo));
+}
+__device__ __forceinline__ double wave_max(double v) {
+    v = max_dpp<0xB1>(v);  /* quad_perm [1,0,3,2] */
+    v = max_dpp<0x4E>(v);  /* quad_perm [2,3,0,1] */
+    v = max_dpp<0x141>(v); /* row_half_mirror */
+    v = max_dpp<0x140>(v); /* row_mirror */
+    const unsigned long long b = __double_as_longlong(v);
+    const auto l = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+    v = fmax(__longlong_as_double(((unsigned long long)h[0] << 32) | l[0]),
+             __longlong_as_double(((unsigned long long)h[1] << 32) | l[1]));
+    const unsigned long long d = __double_as_longlong(v);
+    const auto m = __builtin_amdgcn_permlane32_swap((unsigned)d, (unsigned)d, false, false);
+    const auto n = __builtin_amdgcn_permlane32_swap((unsigned)(d >> 32), (unsigned)(d >> 32), false, false);
+    return fmax(__longlong_as_double(((unsigned long long)n[0] << 32) | m[0]),
+                __longlong_as_double(((unsigned long long)n[1] << 32) | m[1]));
+}
+
+/* entry (m, n) of eps in elimination order, all lanes their own: column 0
+ * goes last (position N - 1), column j > 0 to j - 1; column N is the right-hand
+ * side e_0 */
+struct EpsBlock {
+    int N, nfreq;
+    const double *ReX, *ImX, *qg2;
+    double dfreq;
+    const zd *head;
+    /* element e of the stored lower triangle */
+    __device__ __forceinline__ zd stored(int mat, int e) const {
+        const int q = mat / nfreq, f = mat % nfreq;
+        const size_t src = ((size_t)q * (N * (N + 1) / 2) + e) * nfreq + f;
+        return zd{ReX[src], ImX[src]};
+    }
+    /* entry of row r in position c from the triangle (tri, or null: from memory) */
+    __device__ __forceinline__ zd entry(int mat, const zd *tri, int r, int c) const {
+        if (c >= N) return zd{c == N && r == 0 ? 1.0 : 0.0, 0.0};
+        const int j = c == N - 1 ? 0 : c + 1, m = max(r, j), n = min(r, j), e = m * (m + 1) / 2 + n;
+        zd v = tri ? tri[e] : stored(mat, e);
+        if (r < j) v.y = -v.y;
+        if (r == j) {
+            if (head && r == 0) v = head[mat];
+            else v.x += 1.0;
+            if (qg2) {
+                const double w = dfreq * (mat % nfreq);
+                v.x -= qg2[(size_t)(mat / nfreq) * N + r] / (w * w);
+            }
         }
+        return v;
+    }
+    /* with qg2, w = 0 is an infinite diagonal: no finite inverse */
+    __device__ __forceinline__ bool infinite(int mat) const { return qg2 && mat % nfreq == 0; }
+};
+
+__device__ __forceinline__ void eps_result(int mat, zd u, zd y, zd *epsM, double *elf) {
+    const double du = u.x * u.x + u.y * u.y;
+    const zd t = cmulc(y, u), g{t.x / du, t.y / du}; /* [eps^-1]_00 = y / u */
+    const double den = g.x * g.x + g.y * g.y;
+    epsM[mat] = zd{g.x / den, -g.y / den};
+    elf[mat] = -g.y;
+}
+
+__device__ __forceinline__ double lane_f64(double v, int l) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffff), l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+/* [eps^-1]_00 = x_0 of eps x = e_0, by Gaussian elimination with partial
+ * pivoting of [eps | e_0] in the column order above, so that x_0 is the last
+ * unknown and no back substitution is needed: N^3 / 3 complex products against
+ * the 2 N^3 of the Gauss-Jordan inverse.
+ *
+ * One workgroup of NW waves per (q, f), the matrix in registers: a lane holds
+ * RB rows (lane + 64 b) of its wave's columns w + NW i, i < CW.  In step k the
+ * wave of column k finds the pivot row among the unused ones and publishes the
+ * multipliers of all rows (0 for used ones) and the pivot's index in LDS; after
+ * the step's one barrier every wave updates its columns right of k, the pivot
+ * row's entry read from its lane.  Rows are not swapped.  The two LDS slots
+ * alternate.  Instruction issue bounds it (eight instructions a column and step,
+ * four of them lane reads; some 60 more for the step), so it matters that a
+ * wave works on whole columns: with the rows split over the waves, each finding
+ * the pivot of its own, 1000 matrices of N = 59 took 0.26 ms; with the matrix in
+ * LDS 0.24 ms (LDS bandwidth); Gauss-Jordan in global memory 5.6 ms; this
+ * 0.10 ms.  The stored block has f innermost, so neighbouring f share
+ * lines: each XCD takes a range of f. */
+template <int RB, int NW, int CW>
+__global__ void __launch_bounds__(64 * NW) epsm_reg_kernel(EpsBlock a, zd *epsM, double *elf) {
+    extern __shared__ double eps_sm[];
+    zd *tri = reinterpret_cast<zd *>(eps_sm); /* the stored triangle, then unused */
+    __shared__ zd tbuf[2][RB][64], last[2];
+    __shared__ int pbuf[2];
+    const int mat = xcd_remap(blockIdx.x, gridDim.x), N = a.N;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (a.infinite(mat)) {
+        if (tid == 0) {
+            epsM[mat] = zd{NAN, NAN};
+            elf[mat] = NAN;
+        }
+        return;
+    }
+    const int ne2 = N * (N + 1) / 2;
+    for (int e = tid; e < ne2; e += 64 * NW) tri[e] = a.stored(mat, e);
+    __syncthreads();
+    zd x[CW][RB];
+    bool used[RB];
+#pragma unroll
+    for (int b = 0; b < RB; b++) {
+        const int r = lane + 64 * b;
+        used[b] = r >= N;
+#pragma unroll
+        for (int i = 0; i < CW; i++) {
+            const int c = wave + NW * i;
+            x[i][b] = (r < N && c <= N) ? a.entry(mat, tri, r, c) : zd{0.0, 0.0};
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < CW; i++) {
+        if (NW * i >= N - 1) break;
+        for (int o = 0; o < NW; o++) {
+            const int k = NW * i + o, s = k & 1;
+            if (k >= N - 1) break;
+            if (wave == o) {
+                /* -2: a used row; -1: an entry that is not a number */
+                double bm = -2.0;
+                int bb = 0;
+#pragma unroll
+                for (int b = 0; b < RB; b++) {
+                    const double mag = x[i][b].x * x[i][b].x + x[i][b].y * x[i][b].y;
+                    const double t = used[b] ? -2.0 : (mag >= 0.0 ? mag : -1.0);
+                    bb = t > bm ? b : bb;
+                    bm = fmax(bm, t);
+                }
+                const int pl = __ffsll((long long)__ballot(bm == wave_max(bm))) - 1;
+                const int pb = RB > 1 ? __builtin_amdgcn_readlane(bb, pl) : 0;
+                zd v = x[i][0];
+#pragma unroll
+                for (int b = 1; b < RB; b++)
+                    if (pb == b) v = x[i][b];
+                const zd pv{lane_f64(v.x, pl), lane_f64(v.y, pl)};
+                const double den = 1.0 / (pv.x * pv.x + pv.y * pv.y);
+                const zd ip{pv.x * den, -pv.y * den};
+#pragma unroll
+                for (int b = 0; b < RB; b++)
+                    tbuf[s][b][lane] = (used[b] || (b == pb && lane == pl)) ? zd{0.0, 0.0} : cmul(x[i][b], ip);
+                if (lane == 0) pbuf[s] = pl + 64 * pb;
+            }
+            __syncthreads();
+            const int pr = __builtin_amdgcn_readfirstlane(pbuf[s]), pl = pr & 63, pb = pr >> 6;
+            zd t[RB];
+#pragma unroll
+            for (int b = 0; b < RB; b++) {
+                t[b] = tbuf[s][b][lane];
+                used[b] = used[b] || (b == pb && lane == pl);
+            }
+            auto update = [&](zd(&col)[RB]) {
+                zd v = col[0];
+#pragma unroll
+                for (int b = 1; b < RB; b++)
+                    if (pb == b) v = col[b];
+                const zd p{lane_f64(v.x, pl), lane_f64(v.y, pl)};
+#pragma unroll
+                for (int b = 0; b < RB; b++) {
+                    col[b].x = fma(t[b].y, p.y, fma(-t[b].x, p.x, col[b].x));
+                    col[b].y = fma(-t[b].y, p.x, fma(-t[b].x, p.y, col[b].y));
+                }
+            };
+            if (wave > o) update(x[i]);
+#pragma unroll
+            for (int j = i + 1; j < CW; j++) update(x[j]);
+        }
+    }
+    /* the one row left: columns N - 1 and N */
+#pragma unroll
+    for (int b = 0; b < RB; b++)
+#pragma unroll
+        for (int i = 0; i < CW; i++) {
+            const int c = wave + NW * i;
+            if ((c == N - 1 || c == N) && !used[b]) last[c - (N - 1)] = x[i][b];
+        }
+    __syncthreads();
+    if (tid == 0) eps_result(mat, last[0], last[1], epsM, elf);
+}
+
+/* the same for larger N, one workgroup of 16 waves per (q, f) with its matrix
+ * in the workspace (L2): a wave updates the unused rows r = wave mod 16, a lane
+ * per column */
+__global__ void __launch_bounds__(1024) epsm_ws_kernel(EpsBlock a, zd *work, zd *epsM, double *elf, int mat0) {
+    extern __shared__ int eps_used[]; /* [N] */
+    const int mat = mat0 + xcd_remap(blockIdx.x, gridDim.x), N = a.N, ld = N + 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int NW = 16;
+    if (a.infinite(mat)) {
+        if (tid == 0) {
+            epsM[mat] = zd{NAN, NAN};
+            elf[mat] = NAN;
+        }
+        return;
+    }
+    zd *A = work + (size_t)blockIdx.x * N * ld;
+    for (int r = wave; r < N; r += NW)
+        for (int c = lane; c <= N; c += 64) A[(size_t)r * ld + c] = a.entry(mat, nullptr, r, c);
+    for (int r = tid; r < N; r += 64 * NW) eps_used[r] = 0;
+    __syncthreads();
+    for (int k = 0; k < N; k++) {
+        double bm = -2.0; /* no unused row; -1: an entry that is not a number */
+        int bi = 0;
+        for (int r = lane; r < N; r += 64)
+            if (!eps_used[r]) {
+                const zd v = A[(size_t)r * ld + k];
+                const double mag = v.x * v.x + v.y * v.y, t = mag >= 0.0 ? mag : -1.0;
+                if (t > bm) {
+                    bm = t;
+                    bi = r;
+                }
+            }
+        const int pr = __builtin_amdgcn_readlane(bi, __ffsll((long long)__ballot(bm == wave_max(bm))) - 1);
+        const zd *prow = A + (size_t)pr * ld;
+        if (k + 1 == N) {
+            if (tid == 0) eps_result(mat, prow[N - 1], prow[N], epsM, elf);
+            break;
+        }
+        const zd pv = prow[k];
+        const double den = 1.0 / (pv.x * pv.x + pv.y * pv.y);
+        const zd ip{pv.x * den, -pv.y * den};
+        for (int cb = k + 1; cb <= N; cb += 64) {
+            const int c = cb + lane, cc = min(c, N);
+            const zd p = prow[cc];
+            for (int rb = 0; rb < N; rb += 64) {
+                /* the wave's unused rows of this block of 64, four at a time so
+                 * that their loads are issued together */
+                unsigned long long todo = __ballot(rb + lane < N && rb + lane != pr && (lane & (NW - 1)) == wave &&
+                                                   !eps_used[min(rb + lane, N - 1)]);
+                while (todo) {
+                    int r[4];
+                    zd fr[4], x[4];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        r[u] = todo ? rb + __ffsll((long long)todo) - 1 : -1;
+                        todo &= todo - 1;
+                        const zd *row = A + (size_t)(r[u] < 0 ? pr : r[u]) * ld;
+                        fr[u] = row[k];
+                        x[u] = row[cc];
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const zd t = cmul(fr[u], ip);
+                        x[u].x = fma(t.y, p.y, fma(-t.x, p.x, x[u].x));
+                        x[u].y = fma(-t.y, p.x, fma(-t.x, p.y, x[u].y));
+                        if (r[u] >= 0 && c <= N) A[(size_t)r[u] * ld + c] = x[u];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (tid == 0) eps_used[pr] = 1;
+        __syncthreads();
+    }
+}
+
+constexpr int EPS_REG_N = 127; /* largest N held in registers (two rows a lane, 8 columns in each of 16 waves) */
+
+/* eps_M and ELF of matrices 0 .. nmat - 1 (q, f); the workspace form runs in
+ * launches of as many matrices as its ws_entries hold */
+int launch_epsm(pmx_ctx *c, const EpsBlock &a, int nmat, zd *work, size_t ws_entries, zd *epsM, double *elf) {
+    const size_t per = (size_t)a.N * (a.N + 1);
+    if (a.N <= EPS_REG_N) {
+        const size_t lds = sizeof(zd) * (size_t)a.N * (a.N + 1) / 2;
+        auto go = [&](auto kern, int nw) -> int {
+            if (lds > 65536 - 4608)
+                PMX_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            hipLaunchKernelGGL(kern, dim3(nmat), dim3(64 * nw), lds, c->stream, a, epsM, elf);
+            return 0;
+        };
+        const int rc = a.N <= 15   ? go(epsm_reg_kernel<1, 4, 4>, 4)
+                       : a.N <= 31 ? go(epsm_reg_kernel<1, 4, 8>, 4)
+                       : a.N <= 63 ? go(epsm_reg_kernel<1, 4, 16>, 4)
+                                   : go(epsm_reg_kernel<2, 16, 8>, 16);
+        if (rc) return rc;
+        PMX_CHECK_HIP(hipGetLastError());
+        return 0;
+    }
+    const int chunk = (int)std::min<size_t>(ws_entries / per, (size_t)nmat);
+    for (int m0 = 0; m0 < nmat; m0 += chunk) {
+        hipLaunchKernelGGL(epsm_ws_kernel, dim3(std::min(chunk, nmat - m0)), dim3(1024), sizeof(int) * (size_t)a.N,
+                           c->stream, a, work, epsM, elf, m0);
+        PMX_CHECK_HIP(hipGetLastError());
+    }
+    return 0;
 }
 
 template <class T> __global__ void kkmat_kernel(int nfreq, double dfreq, T *Kk) {
@@ -3473,16 +3757,21 @@ extern "C" int pmx_epsinv(pmx_ctx *c, int nq, int neps, int nfreq, const double 
     DBuf<double> re, im, el;
     DBuf<zd> scr, em, inv;
     int rc;
+    const size_t ws = epsinv ? (size_t)nmat * neps * 2 * neps
+                             : (neps <= EPS_REG_N ? 1 : (size_t)std::min(nmat, 2048) * neps * (neps + 1));
     if ((rc = re.ensure(nblk)) || (rc = im.ensure(nblk)) || (rc = el.ensure(nmat)) || (rc = em.ensure(nmat)) ||
-        (rc = scr.ensure((size_t)nmat * neps * 2 * neps)))
+        (rc = scr.ensure(ws)))
         return rc;
     if (epsinv && (rc = inv.ensure((size_t)nmat * neps * neps))) return rc;
     PMX_CHECK_HIP(hipMemcpyAsync(re.p, ReX, sizeof(double) * nblk, hipMemcpyHostToDevice, st));
     PMX_CHECK_HIP(hipMemcpyAsync(im.p, ImX, sizeof(double) * nblk, hipMemcpyHostToDevice, st));
     {
         Prof pf(c, "epsinv", 8.0 * neps * neps * 2.0 * neps * nmat, 0.0);
-        hipLaunchKernelGGL(epsinv_kernel, dim3(nmat), dim3(256), 0, st, neps, nq, nfreq, re.p, im.p, nullptr, 0.0,
-                           nullptr, scr.p, em.p, el.p, epsinv ? inv.p : nullptr, 0);
+        if (epsinv)
+            hipLaunchKernelGGL(epsinv_kernel, dim3(nmat), dim3(256), 0, st, neps, nfreq, re.p, im.p, scr.p, em.p, el.p,
+                               inv.p);
+        else if ((rc = launch_epsm(c, EpsBlock{neps, nfreq, re.p, im.p, nullptr, 0.0, nullptr}, nmat, scr.p, ws, em.p, el.p)))
+            return rc;
     }
     PMX_CHECK_HIP(hipGetLastError());
     PMX_CHECK_HIP(hipMemcpyAsync(epsM, em.p, sizeof(zd) * nmat, hipMemcpyDeviceToHost, st));
@@ -3512,14 +3801,9 @@ extern "C" int pmx_epsinv_noalloc(pmx_ctx *c, int nq, int neps, int nfreq, const
     zd *ws = noalloc_workspace(c->device);
     if (!ws) return set_error(PMX_ESTATE, "pmx_epsinv_noalloc: the workspace of this device was not set up");
     hipStream_t st = c->stream;
-    const int nmat = nq * nfreq;
-    const int chunk = (int)std::min<size_t>(cap / per_mat, (size_t)nmat);
-    for (int m0 = 0; m0 < nmat; m0 += chunk) {
-        const int nm = std::min(chunk, nmat - m0);
-        hipLaunchKernelGGL(epsinv_kernel, dim3(nm), dim3(256), 0, st, neps, nq, nfreq, dReX, dImX, nullptr, 0.0,
-                           nullptr, ws, reinterpret_cast<zd *>(dEpsM), dElf, nullptr, m0);
-        PMX_CHECK_HIP(hipGetLastError());
-    }
+    if (int rc = launch_epsm(c, EpsBlock{neps, nfreq, dReX, dImX, nullptr, 0.0, nullptr}, nq * nfreq, ws, cap,
+                             reinterpret_cast<zd *>(dEpsM), dElf))
+        return rc;
     PMX_CHECK_HIP(hipStreamSynchronize(st));
     return PMX_OK;
 }
@@ -3555,12 +3839,13 @@ extern "C" int pmx_eps_macro(pmx_ctx *c, int nq, const double *Q, int neps, int 
             qg2[(size_t)q * neps + m] = c0 * c0 * h_eV * h_eV * n2;
         }
     }
+    const size_t ws = neps <= EPS_REG_N ? 1 : (size_t)std::min(nmat, 2048) * neps * (neps + 1);
     DBuf<double> reL, imL, reT, imT, el, qgd;
     DBuf<zd> scr, emL, emT, hd;
     int rc;
     if ((rc = reL.ensure(nblk)) || (rc = imL.ensure(nblk)) || (rc = reT.ensure(nblk)) || (rc = imT.ensure(nblk)) ||
-        (rc = el.ensure(nmat)) || (rc = emL.ensure(nmat)) || (rc = emT.ensure(nmat)) ||
-        (rc = scr.ensure((size_t)nmat * neps * 2 * neps)) || (rc = upload(st, qgd, qg2)))
+        (rc = el.ensure(nmat)) || (rc = emL.ensure(nmat)) || (rc = emT.ensure(nmat)) || (rc = scr.ensure(ws)) ||
+        (rc = upload(st, qgd, qg2)))
         return rc;
     const size_t tblk = 4 * nblk; /* block (i, j) = (1, 1) */
     PMX_CHECK_HIP(hipMemcpyAsync(reL.p, ReX, sizeof(double) * nblk, hipMemcpyHostToDevice, st));
@@ -3578,10 +3863,9 @@ extern "C" int pmx_eps_macro(pmx_ctx *c, int nq, const double *Q, int neps, int 
     if ((rc = upload(st, hd, head))) return rc;
     {
         Prof pf(c, "epsinv", 2.0 * 8.0 * neps * neps * 2.0 * neps * nmat, 0.0);
-        hipLaunchKernelGGL(epsinv_kernel, dim3(nmat), dim3(256), 0, st, neps, nq, nfreq, reL.p, imL.p, nullptr, 0.0,
-                           hd.p, scr.p, emL.p, el.p, nullptr, 0);
-        hipLaunchKernelGGL(epsinv_kernel, dim3(nmat), dim3(256), 0, st, neps, nq, nfreq, reT.p, imT.p, qgd.p, dfreq,
-                           nullptr, scr.p, emT.p, el.p, nullptr, 0);
+        if ((rc = launch_epsm(c, EpsBlock{neps, nfreq, reL.p, imL.p, nullptr, 0.0, hd.p}, nmat, scr.p, ws, emL.p, el.p)) ||
+            (rc = launch_epsm(c, EpsBlock{neps, nfreq, reT.p, imT.p, qgd.p, dfreq, nullptr}, nmat, scr.p, ws, emT.p, el.p)))
+            return rc;
     }
     PMX_CHECK_HIP(hipGetLastError());
     PMX_CHECK_HIP(hipMemcpyAsync(epsM, emL.p, sizeof(zd) * nmat, hipMemcpyDeviceToHost, st));
