@@ -1522,8 +1522,9 @@ __global__ void __launch_bounds__(256, 2) moment_bf3w_kernel(MomArgs2 a, int ngr
 }
 
 /* ------------------------------------------------------------------
- * direct windowed sum (PMX_PREC_DIRECT, triangle, rect): one block per
- * (tile pair, bin); Z[f][pair][256] += sum_t w delta(dE_t - w_f) X X^H
+ * direct windowed sum (PMX_PREC_DIRECT, triangle, rect, principal value):
+ * Z[f][pair][256] = sum_t w kernel(dE_t, w_f) X X^H over the transitions whose
+ * window holds f
  * ------------------------------------------------------------------ */
 struct DirArgs {
     int D, nch, npairs, nbins, wh, nfreq, delta, acc_index;
@@ -1531,10 +1532,11 @@ struct DirArgs {
     const zd *X;              /* sorted FP64 rows */
     const double *es, *ws;    /* sorted dE and weights */
     const int *start;
-    zd *Z;                    /* [nfreq][npairs][256] */
+    zd *Z;                    /* [nfreq][npairs][256], or one such per segment */
     int off_b;                /* bin = f0 + off_b */
     int pv;                   /* principal-value kernels instead of delta: 1 by element class
                                  (chi_LL), 2 the TT kernel for every element (chi_xyz) */
+    int nseg;                 /* segments of the transitions (grid z) */
 };
 
 __device__ double delta_fn(int code, double eps, double x) {
@@ -1548,70 +1550,141 @@ __device__ double delta_fn(int code, double eps, double x) {
     return 0.0;
 }
 
-/* chi_LL's principal-value kernels (src/pmx_chi_copy.cpp:560-577) by the
- * class of the element: 0 = LL (i = j = 0), 1 = LT (one of them 0), 2 = TT */
-__device__ __forceinline__ double pv_fn(int cls, double dE, double w) {
-    const double den = dE * dE - w * w;
-    return cls == 0 ? dE / den : (cls == 1 ? 1.0 / den : 1.0 / dE / den);
-}
-
-__global__ void __launch_bounds__(256) direct_kernel(DirArgs a) {
-    const int pairi = blockIdx.x, b = blockIdx.y;
-    const int t0 = a.start[b], t1 = a.start[b + 1];
-    if (t0 == t1) return;
+/* The sum as a GEMM on FP64 MFMA (16x16x4): frequencies x items times items x
+ * elements, an item being one rank-1 term of a transition (its + or - channel
+ * with SOC).  The products P = X_a conj(X_b) are formed in registers, so an
+ * item costs 4 nfreq real multiply-adds per element instead of the 8 of an
+ * outer product per frequency, and each item is read once per 32 frequencies.
+ * A workgroup owns a tile pair, 32 frequencies and a segment of the items;
+ * wave w the tile rows 4 w .. 4 w + 3 (16 accumulators).  The kernel values of
+ * 16 items are formed together one chunk ahead and shared through LDS.
+ *
+ * chi_LL's principal-value kernels (src/pmx_chi_copy.cpp:560-577) by the class
+ * of the element are dE g (i = j = 0), g (one of them 0) and g / dE with
+ * g = 1 / (dE^2 - w^2): the power of dE goes to the element's side.
+ *
+ * Few tile pairs and frequencies leave the GPU idle, so the items are split
+ * into nseg segments whose sums dir_reduce_kernel adds in a fixed order.  One
+ * workgroup per (tile pair, bin) on the vector ALUs, with an outer product and
+ * an atomic add per frequency, took 2262 us a sum in epsLL of Si with 59 plane
+ * waves, 8^3 k (20,480 transitions), NEPS 9, 101 frequencies; this takes 251
+ * us (32 of 73 TFLOP/s, a fifth of it for frequencies 102-128) and 26 us for
+ * the segments.  Bound by the products' vector work between the MFMAs at two
+ * waves a SIMD. */
+constexpr int DIR_F = 32, DIR_T = 16;
+template <int NI> __global__ void __launch_bounds__(256, 2) direct_kernel(DirArgs a) {
+    __shared__ double kap[2][DIR_T][DIR_F + 2], dk[2][DIR_T][2];
+    const int pairi = blockIdx.x, fa = blockIdx.y * DIR_F, seg = blockIdx.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int kq = lane >> 4, lc = lane & 15;
     int ti, tj;
     tile_pair(pairi, ti, tj);
-    const int r = threadIdx.x / TILE, cc = threadIdx.x % TILE;
-    const int ar = ti * TILE + r, ac = tj * TILE + cc;
-    const int f0 = b - a.off_b;
-    const int fmin = max(0, f0 - a.wh), fmax = min(a.nfreq - 1, f0 + a.wh);
-    const int cls = a.pv == 2 ? 2 : ((ar % 3 == 0 && ac % 3 == 0) ? 0 : ((ar % 3 == 0 || ac % 3 == 0) ? 1 : 2));
-    __shared__ zd xa[32][TILE], xb[32][TILE];
-    __shared__ double ws[3][32];
-    const int per = (a.nch == 1) ? 32 : 16;
-    for (int f = fmin; f <= fmax; f++) {
-        zd acc{0, 0};
-        const double wf = a.w0 + a.df * f;
-        for (int base = t0; base < t1; base += per) {
-            const int cnt = min(per, t1 - base);
-            __syncthreads();
-            for (int e = threadIdx.x; e < 32 * TILE * 2; e += blockDim.x) {
-                int item = e / (2 * TILE), which = (e / TILE) & 1, col = e % TILE;
-                int tl = (a.nch == 1) ? item : item / 2;
-                int ch = (a.nch == 1) ? 0 : (2 * a.acc_index + (item & 1));
-                zd v{0, 0};
-                if (tl < cnt) {
-                    int aa = (which == 0 ? ti : tj) * TILE + col;
-                    if (aa < a.D) v = a.X[((size_t)(base + tl) * a.nch + ch) * a.D + aa];
-                }
-                if (which == 0) xa[item][col] = v; else xb[item][col] = v;
+    /* this segment's items of the transitions with a window that reaches the block */
+    const int b0 = max(0, fa - a.wh + a.off_b), b1 = min(a.nbins - 1, min(fa + DIR_F, a.nfreq) - 1 + a.wh + a.off_b);
+    const long t0 = b0 <= b1 ? a.start[b0] : 0, nt = b0 <= b1 ? a.start[b1 + 1] - t0 : 0;
+    const long i0 = NI * t0 + nt * NI * seg / a.nseg, i1 = NI * t0 + nt * NI * (seg + 1) / a.nseg;
+    const int ac = tj * TILE + lc;
+    const bool cok = ac < a.D;
+    int cls[4], arow[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int ar = ti * TILE + 4 * wave + j;
+        arow[j] = min(ar, a.D - 1);
+        cls[j] = a.pv == 2 ? 2 : ((ar % 3 == 0 && ac % 3 == 0) ? 0 : ((ar % 3 == 0 || ac % 3 == 0) ? 1 : 2));
+    }
+    /* kernel values of the chunk at item ib: two per thread */
+    auto stage = [&](long ib, int s) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int it = (tid >> 5) + 8 * h, fl = tid & (DIR_F - 1);
+            const long i = ib + it;
+            const long t = min(i, i1 - 1) / NI;
+            const double dE = a.es[t], wf = a.w0 + a.df * (fa + fl);
+            double v = 0.0;
+            if (i < i1 && fa + fl < a.nfreq) {
+                const int f0 = int((dE - a.w0) / a.df);
+                const double w = (NI == 2 && (i & 1)) ? -a.ws[t] : a.ws[t];
+                if (abs(f0 - (fa + fl)) <= a.wh)
+                    v = w * (a.pv ? 1.0 / (dE * dE - wf * wf) : delta_fn(a.delta, a.eps, dE - wf));
             }
-            for (int e = threadIdx.x; e < 32 * 3; e += blockDim.x) {
-                const int it = e % 32, k = e / 32;
-                int tl = (a.nch == 1) ? it : it / 2;
-                double w = 0.0;
-                if (tl < cnt && (a.pv || k == 0)) {
-                    w = a.ws[base + tl];
-                    if (a.nch != 1 && (it & 1)) w = -w;
-                    w *= a.pv ? pv_fn(k, a.es[base + tl], wf) : delta_fn(a.delta, a.eps, a.es[base + tl] - wf);
-                }
-                ws[k][it] = w;
-            }
-            __syncthreads();
-            const int nitems = (a.nch == 1) ? cnt : 2 * cnt;
-            const double *wsel = ws[a.pv ? cls : 0];
-            for (int it = 0; it < nitems; it++) {
-                zd p = cmulc(xa[it][r], xb[it][cc]);
-                acc.x += p.x * wsel[it];
-                acc.y += p.y * wsel[it];
+            kap[s][it][fl] = v;
+            if (fl == 0 && a.pv) {
+                dk[s][it][0] = dE;
+                dk[s][it][1] = 1.0 / dE;
             }
         }
-        if (ar < a.D && ac < a.D) {
-            /* bins f0 - wh .. f0 + wh all add into frequency f: atomics */
-            zd *dst = a.Z + ((size_t)f * a.npairs + pairi) * 256 + threadIdx.x;
-            atomicAdd(&dst->x, acc.x);
-            atomicAdd(&dst->y, acc.y);
+    };
+    dx4 accr[2][4], acci[2][4];
+#pragma unroll
+    for (int fb = 0; fb < 2; fb++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) accr[fb][j] = acci[fb][j] = dx4{0, 0, 0, 0};
+    auto load = [&](long i, zd (&xa)[4], zd &xb) {
+        const long ii = min(i, i1 - 1);
+        const size_t row = NI == 1 ? (size_t)ii * a.nch : (size_t)(ii >> 1) * a.nch + 2 * a.acc_index + (ii & 1);
+        const zd *x = a.X + row * a.D;
+#pragma unroll
+        for (int j = 0; j < 4; j++) xa[j] = x[arow[j]];
+        xb = x[min(ac, a.D - 1)];
+    };
+    if (i0 < i1) {
+        zd xa[4], xb;
+        load(i0 + kq, xa, xb);
+        stage(i0, 0);
+        __syncthreads();
+        int s = 0;
+        for (long ib = i0; ib < i1; ib += DIR_T, s ^= 1) {
+            if (ib + DIR_T < i1) stage(ib + DIR_T, s ^ 1);
+#pragma unroll
+            for (int ks = 0; ks < DIR_T / 4; ks++) {
+                const int it = 4 * ks + kq;
+                zd p[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    p[j] = cok ? cmulc(xa[j], xb) : zd{0.0, 0.0};
+                    if (a.pv) {
+                        const double c = cls[j] == 1 ? 1.0 : dk[s][it][cls[j] >> 1];
+                        p[j].x *= c;
+                        p[j].y *= c;
+                    }
+                }
+                load(ib + it + 4, xa, xb); /* the next four items */
+#pragma unroll
+                for (int fb = 0; fb < 2; fb++) {
+                    const double k = kap[s][it][16 * fb + lc];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        accr[fb][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(k, p[j].x, accr[fb][j], 0, 0, 0);
+                        acci[fb][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(k, p[j].y, acci[fb][j], 0, 0, 0);
+                    }
+                }
+            }
+            __syncthreads();
         }
+    }
+    zd *Z = a.Z + (size_t)seg * a.nfreq * a.npairs * 256;
+#pragma unroll
+    for (int fb = 0; fb < 2; fb++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int f = fa + 16 * fb + kq + 4 * v;
+            if (f >= a.nfreq) continue;
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                Z[((size_t)f * a.npairs + pairi) * 256 + (4 * wave + j) * TILE + lc] = zd{accr[fb][j][v], acci[fb][j][v]};
+        }
+}
+
+/* Z = sum of the segments, in order */
+__global__ void __launch_bounds__(256) dir_reduce_kernel(size_t n, int nseg, const zd *part, zd *Z) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        zd s = part[i];
+        for (int g = 1; g < nseg; g++) {
+            const zd p = part[(size_t)g * n + i];
+            s.x += p.x;
+            s.y += p.y;
+        }
+        Z[i] = s;
     }
 }
 
@@ -2822,7 +2895,7 @@ template <class T> int upload(hipStream_t s, DBuf<T> &b, const std::vector<T> &h
 struct ChiWork {
     DBuf<double> Kd, KQd, KWd, evk, dEd, wtd, Ktd, Kkd, Re0, Im0, ReD, ImD; /* evk, vk: [k; k+q] halves */
     DBuf<double> ws, ss, es, qgn;
-    DBuf<zd> vk, Xd, M1, M2, Z1, Z2, wAd, ucd, wSd;
+    DBuf<zd> vk, Xd, M1, M2, Z1, Z2, Zp, wAd, ucd, wSd; /* Zp: the direct sum's segments */
     DBuf<float2> Xf;
     DBuf<float> Ktf, Kkf;
     DBuf<__bf16> kA, kT; /* split-BF16 KK: A rows [Ih | Il | Rh | Rl][M][NFp], K [KhT | KlT][NFc][NFp] */
@@ -3131,9 +3204,9 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
     /* moment buffers and the Taylor table for the current binning */
     auto setup_bins = [&]() -> int {
         int r;
-        if ((r = w.M1.ensure((size_t)nbins * std::max(NT, 1) * npairs * 256))) return r;
+        if (!direct && (r = w.M1.ensure((size_t)nbins * std::max(NT, 1) * npairs * 256))) return r;
         if ((r = w.Z1.ensure((size_t)p->nfreq * npairs * 256))) return r;
-        if (nacc == 2 && (r = w.M2.ensure((size_t)nbins * std::max(NT, 1) * npairs * 256))) return r;
+        if (nacc == 2 && !direct && (r = w.M2.ensure((size_t)nbins * std::max(NT, 1) * npairs * 256))) return r;
         if ((nacc == 2 || pv) && (r = w.Z2.ensure((size_t)p->nfreq * npairs * 256))) return r;
         if (!direct) {
             std::vector<double> Kt;
@@ -3364,17 +3437,35 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
         head("    Solving for Xijmn...");
 
         /* ---- accumulate */
+        /* the per-transition sum: about four workgroups per CU, segments of at
+         * least 64 items and at most 256 MB of partial sums */
+        auto launch_direct = [&](int acc, int pvk, zd *Z) -> int {
+            const int nfb = (p->nfreq + DIR_F - 1) / DIR_F, ni = nch == 1 ? 1 : 2;
+            const size_t zlen = (size_t)p->nfreq * npairs * 256;
+            size_t ns = (4 * (size_t)c->num_cu + npairs * nfb - 1) / ((size_t)npairs * nfb);
+            ns = std::min({ns, ((size_t)ntr * ni + 63) / 64, std::max<size_t>(1, ((size_t)256 << 20) / (sizeof(zd) * zlen))});
+            const int nseg = (int)std::max<size_t>(ns, 1);
+            int rd;
+            if (nseg > 1 && (rd = w.Zp.ensure(zlen * nseg))) return rd;
+            DirArgs da{D, nch, npairs, nbins, wh, p->nfreq, p->delta, acc, p->epsilon, w0, df,
+                       w.Xd.p, w.es.p, w.ws.p, w.start.p, nseg > 1 ? w.Zp.p : Z, off_b, pvk, nseg};
+            hipLaunchKernelGGL(ni == 1 ? direct_kernel<1> : direct_kernel<2>, dim3(npairs, nfb, nseg), dim3(256), 0, st, da);
+            PMX_CHECK_HIP(hipGetLastError());
+            if (nseg > 1)
+                hipLaunchKernelGGL(dir_reduce_kernel, dim3((unsigned)std::min<size_t>((zlen + 255) / 256, 4096)), dim3(256), 0,
+                                   st, zlen, nseg, w.Zp.p, Z);
+            PMX_CHECK_HIP(hipGetLastError());
+            return 0;
+        };
         for (int acc = 0; acc < nacc; acc++) {
             DBuf<zd> &Z = acc == 0 ? w.Z1 : w.Z2;
             DBuf<zd> &M = acc == 0 ? w.M1 : w.M2;
-            if (direct || ntr_sz == 0)
+            if (ntr_sz == 0)
                 PMX_CHECK_HIP(hipMemsetAsync(Z.p, 0, sizeof(zd) * (size_t)p->nfreq * npairs * 256, st));
             if (ntr_sz == 0) continue;
             if (direct) {
-                DirArgs da{D, nch, npairs, nbins, wh, p->nfreq, p->delta, acc, p->epsilon, w0, df,
-                           w.Xd.p, w.es.p, w.ws.p, w.start.p, Z.p, off_b, 0};
                 Prof pf(c, "direct", 8.0 * 9.0 * ne2 * ntr * std::min(2 * wh + 1, p->nfreq) * nacc, 0.0);
-                hipLaunchKernelGGL(direct_kernel, dim3(npairs, nbins), dim3(256), 0, st, da);
+                if ((rc = launch_direct(acc, 0, Z.p))) return rc;
             } else {
                 /* PMX_KSUM=fp32 sums the k-range partials of the FP32 paths in FP32
                  * (to measure what the FP64 cross-k reduction buys) */
@@ -3500,14 +3591,12 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
         }
         if (pv) {
             /* chi_LL's principal-value sums into Z2 */
-            PMX_CHECK_HIP(hipMemsetAsync(w.Z2.p, 0, sizeof(zd) * (size_t)p->nfreq * npairs * 256, st));
             if (ntr > 0) {
-                DirArgs da{D, nch, npairs, nbins, wh, p->nfreq, p->delta, 0, p->epsilon, w0, df,
-                           w.Xd.p, w.es.p, w.ws.p, w.start.p, w.Z2.p, off_b, xyz ? 2 : 1};
                 Prof pf(c, "direct_pv", 8.0 * 9.0 * ne2 * ntr * p->nfreq, 0.0);
-                hipLaunchKernelGGL(direct_kernel, dim3(npairs, nbins), dim3(256), 0, st, da);
+                if ((rc = launch_direct(0, xyz ? 2 : 1, w.Z2.p))) return rc;
+            } else {
+                PMX_CHECK_HIP(hipMemsetAsync(w.Z2.p, 0, sizeof(zd) * (size_t)p->nfreq * npairs * 256, st));
             }
-            PMX_CHECK_HIP(hipGetLastError());
         }
 
         /* ---- scale + pack (+ KK) */
