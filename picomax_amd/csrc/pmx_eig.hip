@@ -3764,6 +3764,16 @@ int tridiag_generic(pmx_ctx *c, EigArgs &a, bool real, bool lds_matrix, int grid
                              }});
         };
         add("ctile6", 6, tridiag_tile_cplx_kernel<6, 2>);
+        /* the default, for batches too small to time and untimed runs: register
+         * tiles hide none of a step's barriers below five of them.  A call of
+         * bands for 64 matrices, three_stream / fused / ctile6: N 15 114 / 108 /
+         * 119 us, N 30 217 / 207 / 208, N 51 413 / 382 / 273, N 89 1034 / 952 /
+         * 462, N 130 2113 / 1915 / 697 */
+        if (lds_matrix) {
+            const char *pref = N >= 30 ? "ctile6" : "fused";
+            for (size_t i = 1; i < cands.size(); i++)
+                if (std::strcmp(cands[i].name, pref) == 0) std::swap(cands[0], cands[i]);
+        }
     }
     const std::string key = std::string(real ? "tridiag real" : "tridiag complex") +
                             (lds_matrix ? " lds N=" : " global N=") + std::to_string(N);

@@ -114,3 +114,22 @@ def test_vectors_of_large_bases(args, gcut2, nk):
         assert np.abs(ev[k] - w[:24]).max() < 1e-10
         assert np.abs(H @ z - z * ev[k]).max() < 1e-12 * np.abs(w).max()
     ctx.close()
+
+
+# complex bases in LDS, on both sides of the size where the default changes
+# (29 / 30) and around multiples of the 6 x 6 tile
+@pytest.mark.parametrize("gcut2,us", [(0.5, {3: 0.01}), (3.1, {3: 0.01}), (4.1, {3: 0.01}), (8.1, None), (8.1, {3: 0.01}),
+                                      (11.1, None), (11.1, {3: 0.01}), (19.1, None), (16.1, {3: 0.01})])
+@pytest.mark.parametrize("nk", [1, 5])
+def test_vectors_of_small_complex_bases(gcut2, us, nk):
+    ctx, s = _pair(VG_AB, gcut2, us=us)
+    K = np.random.default_rng(7).uniform(-0.5, 0.5, (nk, 3))
+    n = s.hamiltonian(K[0]).shape[0] // (1 if us else 2)
+    nb = min(n, 12) if us else 2 * min(n, 12)
+    ev, vec = ctx.eig(K, nb, vectors=True)
+    for k in range(nk):
+        H = s.hamiltonian(K[k])
+        V = vec[k].T
+        assert np.abs(ev[k] - np.linalg.eigvalsh(H)[:nb]).max() < 1e-10
+        assert np.abs(H @ V - V * ev[k]).max() < 1e-9
+    ctx.close()
