@@ -1644,31 +1644,38 @@ __global__ void __launch_bounds__(EIG_THREADS) tridiag_full_real_kernel(EigArgs 
  *   v, tau, beta from x (every wave reduces |x|^2 itself, bit-identically);
  *   tile (I, J) writes A_IJ v_J into slot (I, J) and A_IJ^T v_I into (J, I);
  *   row r sums its slots: p = tau A v;  w = p - (tau/2)(p.v) v;
- *   A_IJ -= v_I w_J^T + w_I v_J^T; the tiles of column k+1 write it out. */
+ *   A_IJ -= v_I w_J^T + w_I v_J^T; the tiles of column k+1 write it out.
+ *
+ * Bound by the latency of a step's chain (about 430 vector instructions, 60
+ * LDS accesses, two reductions): the vector ALUs are busy 39% of the time at
+ * three workgroups per CU.  So what limits the workgroups per CU counts: a
+ * wave ends when its last tile and row retire (1.8 of 4 are alive on average
+ * at N = 137), and LDS holds nothing that can go to memory at once
+ * (reflectors, d, e) or be kept as a running value (the bounds): 52.8 -> 31.3
+ * KB at N = 137, five workgroups per CU instead of three.  27,648 matrices of
+ * order 137: 13.5 -> 9.0 ms; 2,000: 1.12 -> 0.83 ms. */
 constexpr int TILE_MAX_THREADS = 256;
 
 /* TT: tile edge; NB: block rows (NB TT >= N; the rows past N are zero
  * padding), a compile-time count so that every per-step loop over blocks is
- * unrolled with constant offsets; TS = TT + 2: LDS stride of one block of a
+ * unrolled with constant offsets; TS: odd LDS stride of one block of a
  * vector (bank spread); WPE: waves per SIMD the register budget is cut for */
 template <int TT, int NB, int WPE>
 __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kernel(EigArgs a) {
     static_assert(NB * (NB + 1) / 2 <= TILE_MAX_THREADS && NB * TT <= 192, "tile grid too large");
-    constexpr int TS = TT + 2;
-    constexpr int nblk = NB, NR = NB * TT, nvp = NB * TS, nblkp = NB | 1;
+    constexpr int TS = TT | 1;
+    constexpr int nblk = NB, NR = NB * TT, nvp = NB * TS + 1, nblkp = NB | 1;
     /* at 3 waves per SIMD the step orders its loads to keep the live
      * registers within budget; at 2 it issues each phase's loads together */
     constexpr bool LEAN = WPE >= 3;
     auto tvi = [](int r) { return (r / TT) * TS + (r % TT); };
     extern __shared__ double smem_d[];
     const int N = a.N;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     double *xk0 = smem_d, *xk1 = xk0 + nvp, *pp = xk1 + nvp;
     double *vw = pp + nvp + (size_t)wave * nvp;                       /* this wave's copy of v */
     double *part = pp + nvp + (size_t)(blockDim.x >> 6) * nvp;        /* [contributing block C][row block R][TS] */
-    double *dd = part + (size_t)nblk * nblkp * TS;                    /* [N] */
-    double *ee = dd + N, *tt = ee + N;
-    double *ring = tt + N; /* [8][NR]: reflectors of the last 8 steps, stored to global together */
+    double *bnd = part + (size_t)nblk * nblkp * TS; /* running bounds of T, max e^2, the last |e| */
     const int ntile = nblk * (nblk + 1) / 2;
     const int mat = blockIdx.x;
     const size_t P = (size_t)N * (N + 1) / 2;
@@ -1690,7 +1697,8 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
      * tiles that do.  A wave has work at step k while one of its tiles is
      * active (block column J >= (k+1)/TT, J <= Jmax of its first tile) or
      * one of its rows is not yet eliminated (row NR-1-64w >= k); after that it
-     * only meets the barriers, so retired waves cost no VALU time. */
+     * ends, which gives its registers to the next workgroup (a barrier waits
+     * for the waves that are left). */
     const int rrow = NR - 1 - tid; /* this thread's row-sum / reflector row (< 0: none) */
     int wave_last;
     {
@@ -1739,10 +1747,10 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
     /* Each phase of a step issues its LDS loads together and unconditionally
      * (values out of range discarded by selects), so it waits for LDS once;
      * loads under per-lane branches would each wait a full round trip.  Rows
-     * past NR use the padding slot TT of block 0, which no tile reads. */
+     * past NR use the slot behind the last block, which no tile reads. */
     int voc[3];
 #pragma unroll
-    for (int q = 0; q < 3; q++) voc[q] = (lane + 64 * q < NR) ? voff[q] : TT;
+    for (int q = 0; q < 3; q++) voc[q] = (lane + 64 * q < NR) ? voff[q] : NB * TS;
     const int rr = rrow >= 0 ? rrow : 0;
     const double *rslot = part + (size_t)(rr / TT) * TS + rr % TT; /* slot C of row rr: rslot[C nblkp TS] */
     const int tvr = tvi(rr);
@@ -1754,12 +1762,7 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
         const int cur = (TT % 2 == 0) ? ((s + 1) & 1) : (k & 1); /* k & 1, a constant when TT is even */
         const double *x = cur ? xk1 : xk0;
         double *xn = cur ? xk0 : xk1;
-        if (k > wave_last) { /* retired wave: the step's barriers only */
-            __syncthreads();
-            __syncthreads();
-            __syncthreads();
-            continue;
-        }
+        if (k > wave_last) return;
         /* Householder vector of column k; every wave forms it in its own copy */
         double xq[3];
 #pragma unroll
@@ -1856,15 +1859,20 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
                 }
                 pp[tvr] = (rrow > k && rrow < N) ? p * tau : 0.0;
                 /* reflector of this step */
-                if (vref && rrow >= k + 2 && rrow < N) ring[(k & 7) * NR + rrow] = vr;
+                if (vref && rrow >= k + 2 && rrow < N) (vref + (pk(k + 2, k, N) - k - 2))[(unsigned)rrow] = vr;
             } else if (vref && rrow >= k + 2 && rrow < N) {
-                ring[(k & 7) * NR + rrow] = 0.0; /* tau = 0: the step is the identity */
+                (vref + (pk(k + 2, k, N) - k - 2))[(unsigned)rrow] = 0.0; /* tau = 0: the step is the identity */
             }
         }
         if (tid == 0) {
-            dd[k] = xdiag;
-            ee[k] = beta;
-            tt[k] = tau;
+            a.dS[(size_t)k * a.nmat + mat] = xdiag;
+            a.eS[(size_t)k * a.nmat + mat] = beta;
+            if (a.tauv) reinterpret_cast<double *>(a.tauv)[(size_t)mat * N + k] = tau;
+            const double ep = k > 0 ? bnd[3] : 0.0, off = ep + fabs(beta);
+            bnd[0] = fmin(k > 0 ? bnd[0] : xdiag, xdiag - off);
+            bnd[1] = fmax(k > 0 ? bnd[1] : xdiag, xdiag + off);
+            bnd[2] = fmax(k > 0 ? bnd[2] : 0.0, beta * beta);
+            bnd[3] = fabs(beta);
         }
         __syncthreads(); /* (2) p */
         if (tau != 0.0) {
@@ -1945,39 +1953,18 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
             }
         }
         __syncthreads(); /* (3) next column */
-        if (vref && wave == 0 && ((k & 7) == 7 || k + 2 == N)) {
-            /* reflector columns k0..k (rows kk+2..N-1 of column kk are contiguous);
-             * wave 0 is active at every step */
-            const int k0 = k & ~7;
-            for (int kk = k0; kk <= k; kk++) {
-                const int len = N - kk - 2;
-                double *dst = vref + pk(kk + 2, kk, N);
-                for (int i = lane; i < len; i += 64) dst[i] = ring[(kk & 7) * NR + kk + 2 + i];
-            }
-        }
     }
-    }
-    if (tid == 0) dd[N - 1] = ((N & 1) ? xk0 : xk1)[tvi(N - 1)]; /* column N-1 was written at step N-2 */
-    __syncthreads();
-    for (int i = tid; i < N; i += blockDim.x) {
-        a.dS[(size_t)i * a.nmat + mat] = dd[i];
-        a.eS[(size_t)i * a.nmat + mat] = (i + 1 < N) ? ee[i] : 0.0;
-        if (a.tauv) reinterpret_cast<double *>(a.tauv)[(size_t)mat * N + i] = (i + 1 < N) ? tt[i] : 0.0;
     }
     if (tid == 0) {
-        double gl = dd[0], gu = dd[0], emax2 = 0.0;
-        for (int i = 0; i < N; i++) {
-            const double di = dd[i];
-            double off = (i > 0 ? fabs(ee[i - 1]) : 0.0) + (i + 1 < N ? fabs(ee[i]) : 0.0);
-            gl = fmin(gl, di - off);
-            gu = fmax(gu, di + off);
-            if (i + 1 < N) emax2 = fmax(emax2, ee[i] * ee[i]);
-        }
-        double tnorm = fmax(fabs(gl), fabs(gu));
-        gl -= 2.0 * DBL_EPSILON * tnorm * N + 1e-300;
-        gu += 2.0 * DBL_EPSILON * tnorm * N + 1e-300;
-        a.gb[4 * mat] = gl;
-        a.gb[4 * mat + 1] = gu;
+        const double dn = ((N & 1) ? xk0 : xk1)[tvi(N - 1)]; /* column N-1 was written at step N-2 */
+        const double off = N > 1 ? bnd[3] : 0.0, emax2 = N > 1 ? bnd[2] : 0.0;
+        const double gl = fmin(N > 1 ? bnd[0] : dn, dn - off), gu = fmax(N > 1 ? bnd[1] : dn, dn + off);
+        a.dS[(size_t)(N - 1) * a.nmat + mat] = dn;
+        a.eS[(size_t)(N - 1) * a.nmat + mat] = 0.0;
+        if (a.tauv) reinterpret_cast<double *>(a.tauv)[(size_t)mat * N + N - 1] = 0.0;
+        const double tnorm = fmax(fabs(gl), fabs(gu));
+        a.gb[4 * mat] = gl - (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
+        a.gb[4 * mat + 1] = gu + (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
         a.gb[4 * mat + 2] = DBL_MIN * fmax(1.0, emax2);
         a.gb[4 * mat + 3] = tnorm;
     }
@@ -3947,9 +3934,9 @@ static int eig_device_run(pmx_ctx *c, int nmat, const double *dKpts, int nb, int
                 return (std::max(nb_ * (nb_ + 1) / 2, nb_ * tt) + 63) / 64 * 64;
             };
             auto tile_lds = [&](int tt) {
-                const int nb_ = tile_nb(tt), ts = tt + 2;
-                return sizeof(double) * ((3 + tile_threads(tt) / 64) * (size_t)nb_ * ts +
-                                         (size_t)nb_ * (nb_ | 1) * ts + 3 * (size_t)N + 8 * (size_t)nb_ * tt);
+                const int nb_ = tile_nb(tt), ts = tt | 1;
+                return sizeof(double) *
+                       ((3 + tile_threads(tt) / 64) * ((size_t)nb_ * ts + 1) + (size_t)nb_ * (nb_ | 1) * ts + 4);
             };
             /* real path: the register-tiled kernel (7x7 or 8x8 tiles, 2 or 3
              * waves per SIMD) and the full-LDS kernel where they fit, chosen
