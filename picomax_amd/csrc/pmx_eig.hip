@@ -243,6 +243,25 @@ __device__ __forceinline__ void write_bounds(const EigArgs &a, int N, int mat, c
     }
 }
 
+/* the same kept running as d_k and e_k come, by one thread: lower and upper
+ * bound, max e^2 and the last |e| */
+__device__ __forceinline__ void run_bounds(double *b, int k, double d, double e) {
+    const double off = (k > 0 ? b[3] : 0.0) + fabs(e);
+    b[0] = fmin(k > 0 ? b[0] : d, d - off);
+    b[1] = fmax(k > 0 ? b[1] : d, d + off);
+    b[2] = fmax(k > 0 ? b[2] : 0.0, e * e);
+    b[3] = fabs(e);
+}
+__device__ __forceinline__ void last_bounds(const EigArgs &a, int N, int mat, const double *b, double d) {
+    const double off = N > 1 ? b[3] : 0.0, emax2 = N > 1 ? b[2] : 0.0;
+    const double gl = fmin(N > 1 ? b[0] : d, d - off), gu = fmax(N > 1 ? b[1] : d, d + off);
+    const double tnorm = fmax(fabs(gl), fabs(gu));
+    a.gb[4 * mat] = gl - (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
+    a.gb[4 * mat + 1] = gu + (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
+    a.gb[4 * mat + 2] = DBL_MIN * fmax(1.0, emax2);
+    a.gb[4 * mat + 3] = tnorm;
+}
+
 /* deterministic start vector entry in [-1, 1) */
 __device__ __forceinline__ double hash_unit(unsigned a, unsigned b) {
     unsigned h = a * 0x9E3779B1u ^ (b + 0x7F4A7C15u) * 0x85EBCA77u;
@@ -1868,11 +1887,7 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
             a.dS[(size_t)k * a.nmat + mat] = xdiag;
             a.eS[(size_t)k * a.nmat + mat] = beta;
             if (a.tauv) reinterpret_cast<double *>(a.tauv)[(size_t)mat * N + k] = tau;
-            const double ep = k > 0 ? bnd[3] : 0.0, off = ep + fabs(beta);
-            bnd[0] = fmin(k > 0 ? bnd[0] : xdiag, xdiag - off);
-            bnd[1] = fmax(k > 0 ? bnd[1] : xdiag, xdiag + off);
-            bnd[2] = fmax(k > 0 ? bnd[2] : 0.0, beta * beta);
-            bnd[3] = fabs(beta);
+            run_bounds(bnd, k, xdiag, beta);
         }
         __syncthreads(); /* (2) p */
         if (tau != 0.0) {
@@ -1957,16 +1972,10 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_real_kerne
     }
     if (tid == 0) {
         const double dn = ((N & 1) ? xk0 : xk1)[tvi(N - 1)]; /* column N-1 was written at step N-2 */
-        const double off = N > 1 ? bnd[3] : 0.0, emax2 = N > 1 ? bnd[2] : 0.0;
-        const double gl = fmin(N > 1 ? bnd[0] : dn, dn - off), gu = fmax(N > 1 ? bnd[1] : dn, dn + off);
         a.dS[(size_t)(N - 1) * a.nmat + mat] = dn;
         a.eS[(size_t)(N - 1) * a.nmat + mat] = 0.0;
         if (a.tauv) reinterpret_cast<double *>(a.tauv)[(size_t)mat * N + N - 1] = 0.0;
-        const double tnorm = fmax(fabs(gl), fabs(gu));
-        a.gb[4 * mat] = gl - (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
-        a.gb[4 * mat + 1] = gu + (2.0 * DBL_EPSILON * tnorm * N + 1e-300);
-        a.gb[4 * mat + 2] = DBL_MIN * fmax(1.0, emax2);
-        a.gb[4 * mat + 3] = tnorm;
+        last_bounds(a, N, mat, bnd, dn);
     }
 }
 
@@ -2019,49 +2028,85 @@ __device__ __noinline__ zd herm_elem(const EigArgs &a, const double *Kv, int r, 
     return (r >= c) ? h_elem<zd>(a, Kv, r, c) : cj(h_elem<zd>(a, Kv, c, r));
 }
 
-template <int TT, int WPE>
+template <int TT, int QN, int WPE>
 __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kernel(EigArgs a, int nblk) {
-    constexpr int TS = TT + 1;
+    constexpr int TS = TT | 1;
     auto tvi = [](int r) { return (r / TT) * TS + (r % TT); };
     extern __shared__ double smem_d[];
     const int N = a.N, NR = nblk * TT;
-    const int nvp = nblk * TS, nblkp = nblk | 1;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    zd *xk0 = reinterpret_cast<zd *>(smem_d), *xk1 = xk0 + nvp, *pp = xk1 + nvp;
-    zd *vw = pp + nvp + (size_t)wave * nvp;                        /* this wave's copy of v */
-    zd *part = pp + nvp + (size_t)(blockDim.x >> 6) * nvp;         /* [contributing block C][row block R][TS] */
-    zd *tt = part + (size_t)nblk * nblkp * TS;                     /* [N] */
-    double *dd = reinterpret_cast<double *>(tt + N), *ee = dd + N;  /* [N] each */
+    const int nvp = nblk * TS + 1, nblkp = nblk | 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    zd *xk0 = reinterpret_cast<zd *>(smem_d), *xk1 = xk0 + nvp;
+    zd *vw = xk1 + nvp + (size_t)wave * nvp;                       /* this wave's copy of v */
+    zd *part = xk1 + nvp + (size_t)(blockDim.x >> 6) * nvp;        /* [contributing block C][row block R][TS] */
+    double *bnd = reinterpret_cast<double *>(part + (size_t)nblk * nblkp * TS); /* as in the real kernel */
     const int ntile = nblk * (nblk + 1) / 2;
     const int mat = blockIdx.x;
     const size_t P = (size_t)N * (N + 1) / 2;
 
     /* tile of this thread: the m-th group holds block column J = nblk-1-m, rows I = J..nblk-1 */
+    auto group = [](int t) {
+        int m = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+        while (m * (m + 1) / 2 > t) m--;
+        while ((m + 1) * (m + 2) / 2 <= t) m++;
+        return m;
+    };
     int I = 0, J = 0;
     const bool has_tile = tid < ntile;
     if (has_tile) {
-        int m = (int)((sqrt(8.0 * tid + 1.0) - 1.0) * 0.5);
-        while (m * (m + 1) / 2 > tid) m--;
-        while ((m + 1) * (m + 2) / 2 <= tid) m++;
+        const int m = group(tid);
         J = nblk - 1 - m;
         I = J + (tid - m * (m + 1) / 2);
     }
     const bool diag = I == J;
     const int r0 = I * TT, c0 = J * TT;
     const int ib = I * TS, jb = J * TS;
+    /* rows in reverse, and a wave ends when its last tile and the block of its
+     * last row are eliminated (as in the real kernel) */
+    const int rrow = NR - 1 - tid, rr = max(rrow, 0), tvr = tvi(rr);
+    const zd *rslot = part + (size_t)(rr / TT) * TS + rr % TT;
+    int wave_last;
+    {
+        const int t0 = wave * 64;
+        const int last_tile = t0 < ntile ? TT * (nblk - group(t0)) - 1 : -1;
+        const int last_row = NR - 1 - t0 >= 0 ? (NR - 1 - t0) / TT * TT + TT - 1 : -1;
+        wave_last = __builtin_amdgcn_readfirstlane(max(last_tile, last_row));
+    }
+    int voc[QN]; /* rows lane + 64 q; those past NR use the slot behind the last block */
+#pragma unroll
+    for (int q = 0; q < QN; q++) voc[q] = lane + 64 * q < NR ? tvi(lane + 64 * q) : nblk * TS;
     const double Kv[3] = {a.K[3 * mat], a.K[3 * mat + 1], a.K[3 * mat + 2]};
     zd *vref = a.vref ? reinterpret_cast<zd *>(a.vref) + (size_t)mat * P : nullptr;
 
     zd A[TT][TT];
+    if (a.mode == HM_SPATIAL_COMPLEX) {
+        /* loads of a row together; the upper triangle from the lower one */
 #pragma unroll
-    for (int i = 0; i < TT; i++)
+        for (int i = 0; i < TT; i++) {
+            const int r = r0 + i;
 #pragma unroll
-        for (int j = 0; j < TT; j++) {
-            const int r = r0 + i, c = c0 + j;
-            zd h = zd{0.0, 0.0};
-            if (has_tile && r < N && c < N) h = herm_elem(a, Kv, r, c);
-            A[i][j] = h;
+            for (int j = 0; j < TT; j++) {
+                const int c = c0 + j;
+                A[i][j] = zd{0.0, 0.0};
+                if (has_tile && r < N && c < N) A[i][j] = a.Vpair[(size_t)max(r, c) * a.npw + min(r, c)];
+                if (r < c) A[i][j].y = -A[i][j].y;
+            }
         }
+        if (diag)
+#pragma unroll
+            for (int i = 0; i < TT; i++)
+                if (has_tile && r0 + i < N) A[i][i] = h_elem<zd>(a, Kv, r0 + i, r0 + i);
+    } else {
+#pragma unroll
+        for (int i = 0; i < TT; i++)
+#pragma unroll
+            for (int j = 0; j < TT; j++) {
+                const int r = r0 + i, c = c0 + j;
+                zd h = zd{0.0, 0.0};
+                if (has_tile && r < N && c < N) h = herm_elem(a, Kv, r, c);
+                A[i][j] = h;
+            }
+    }
     if (has_tile && J == 0)
 #pragma unroll
         for (int i = 0; i < TT; i++) xk0[(ib + i)] = A[i][0];
@@ -2071,13 +2116,23 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kerne
     for (int s = 0; s < TT; s++) {
         const int k = kb1 + s - 1;
         if (k < 0 || k + 1 >= N) continue;
+        if (k > wave_last) return;
         const int cur = (TT % 2 == 0) ? ((s + 1) & 1) : (k & 1);
         const zd *x = cur ? xk1 : xk0;
         zd *xn = cur ? xk0 : xk1;
-        double s2 = 0.0;
-        for (int r = k + 2 + lane; r < N; r += 64) s2 += nrm2(x[tvi(r)]);
-        s2 = wave_sum_full(s2);
+        zd *pp = cur ? xk1 : xk0; /* p takes the place of x, which is not read after the first barrier */
+        zd xq[QN];
+#pragma unroll
+        for (int q = 0; q < QN; q++) xq[q] = x[voc[q]];
         const zd alpha = x[tvi(k + 1)];
+        const double xdiag = x[tvi(k)].x;
+        double s2 = 0.0;
+#pragma unroll
+        for (int q = 0; q < QN; q++) {
+            const int r = lane + 64 * q;
+            s2 = (r >= k + 2 && r < N) ? fma(xq[q].y, xq[q].y, fma(xq[q].x, xq[q].x, s2)) : s2;
+        }
+        s2 = wave_sum_full(s2);
         double beta;
         zd tau, scal;
         if (s2 == 0.0 && alpha.y == 0.0) {
@@ -2086,16 +2141,17 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kerne
             scal = zd{0.0, 0.0};
         } else {
             beta = -copysign(sqrt(nrm2(alpha) + s2), alpha.x);
-            tau = cdiv(zd{beta, 0.0} - alpha, zd{beta, 0.0});
+            tau = zd{(beta - alpha.x) / beta, -alpha.y / beta};
             scal = cdiv(zd{1.0, 0.0}, alpha - zd{beta, 0.0});
         }
         const bool tnz = tau.x != 0.0 || tau.y != 0.0;
         const int cmin = (k + 1) / TT;
         const bool active = has_tile && J >= cmin && tnz;
         if (tnz) {
-            for (int r = cmin * TT + lane; r < NR; r += 64) {
-                const zd xr = x[tvi(r)];
-                vw[tvi(r)] = (r == k + 1) ? zd{1.0, 0.0} : ((r > k + 1 && r < N) ? xr * scal : zd{0.0, 0.0});
+#pragma unroll
+            for (int q = 0; q < QN; q++) {
+                const int r = lane + 64 * q;
+                vw[voc[q]] = (r == k + 1) ? zd{1.0, 0.0} : ((r > k + 1 && r < N) ? xq[q] * scal : zd{0.0, 0.0});
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -2112,7 +2168,7 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kerne
                 for (int i = 0; i < TT; i++) {
                     zd pi = zd{0.0, 0.0};
 #pragma unroll
-                    for (int j = 0; j < TT; j++) pi += A[i][j] * vJ[j];
+                    for (int j = 0; j < TT; j++) pi = mad(pi, A[i][j], vJ[j]);
                     sI[i] = pi;
                 }
             }
@@ -2125,36 +2181,57 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kerne
                 for (int j = 0; j < TT; j++) {
                     zd pj = zd{0.0, 0.0};
 #pragma unroll
-                    for (int i = 0; i < TT; i++) pj += cj(A[i][j]) * vI[i];
+                    for (int i = 0; i < TT; i++) pj = madc(pj, A[i][j], vI[i]);
                     sJ[j] = pj;
                 }
             }
         }
         __syncthreads(); /* (1) partials */
-        if (tnz && tid < NR) {
-            const int r = tid, R = r / TT, i = r % TT;
-            zd p = zd{0.0, 0.0};
-            if (r > k && r < N) {
-                const zd *col = part + (size_t)R * TS + i;
-                for (int C = cmin; C < nblk; C++) p += col[(size_t)C * nblkp * TS];
-                p = tau * p;
+        if (rrow >= 0) {
+            const bool live = rrow > k && rrow < N;
+            if (tnz) {
+                const zd vr = vw[tvr];
+                zd p = zd{0.0, 0.0};
+                int C = cmin;
+                for (; C + 4 <= nblk; C += 4) {
+                    zd sl[4];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) sl[u] = rslot[(size_t)(C + u) * nblkp * TS];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) p += sl[u];
+                }
+                for (; C < nblk; C++) p += rslot[(size_t)C * nblkp * TS];
+                pp[tvr] = live ? tau * p : zd{0.0, 0.0};
+                if (vref && live && rrow > k + 1) (vref + (pk(k + 2, k, N) - k - 2))[(unsigned)rrow] = vr;
+            } else if (vref && live && rrow > k + 1) {
+                (vref + (pk(k + 2, k, N) - k - 2))[(unsigned)rrow] = zd{0.0, 0.0}; /* tau = 0: the identity */
             }
-            pp[tvi(r)] = p;
         }
-        /* reflector of this step (zero when tau = 0: the step is the identity) */
-        if (vref && tid >= k + 2 && tid < N) vref[pk(tid, k, N)] = tnz ? vw[tvi(tid)] : zd{0.0, 0.0};
         if (tid == 0) {
-            dd[k] = x[tvi(k)].x;
-            ee[k] = beta;
-            tt[k] = tau;
+            a.dS[(size_t)k * a.nmat + mat] = xdiag;
+            a.eS[(size_t)k * a.nmat + mat] = beta;
+            if (a.tauv) reinterpret_cast<zd *>(a.tauv)[(size_t)mat * N + k] = tau;
+            run_bounds(bnd, k, xdiag, beta);
         }
         __syncthreads(); /* (2) p */
         if (tnz) {
             double pr = 0.0, pim = 0.0;
-            for (int r = k + 1 + lane; r < N; r += 64) {
-                const zd cv = cj(pp[tvi(r)]) * vw[tvi(r)];
-                pr += cv.x;
-                pim += cv.y;
+            {
+                zd pq[QN], vq[QN];
+#pragma unroll
+                for (int q = 0; q < QN; q++) {
+                    pq[q] = pp[voc[q]];
+                    vq[q] = vw[voc[q]];
+                }
+#pragma unroll
+                for (int q = 0; q < QN; q++) {
+                    const int r = lane + 64 * q;
+                    const zd c = madc(zd{pr, pim}, pq[q], vq[q]);
+                    if (r >= k + 1 && r < N) {
+                        pr = c.x;
+                        pim = c.y;
+                    }
+                }
             }
             pr = wave_sum_full(pr);
             pim = wave_sum_full(pim);
@@ -2164,24 +2241,24 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kerne
                 {
                     zd u[TT], z[TT];
 #pragma unroll
-                    for (int j = 0; j < TT; j++) z[j] = cj(pp[(jb + j)] + al * vw[(jb + j)]);
+                    for (int j = 0; j < TT; j++) z[j] = cj(mad(pp[(jb + j)], al, vw[(jb + j)]));
 #pragma unroll
                     for (int i = 0; i < TT; i++) u[i] = vw[(ib + i)];
 #pragma unroll
                     for (int i = 0; i < TT; i++)
 #pragma unroll
-                        for (int j = 0; j < TT; j++) A[i][j] -= u[i] * z[j];
+                        for (int j = 0; j < TT; j++) A[i][j] = msub(A[i][j], u[i], z[j]);
                 }
                 {
                     zd u[TT], z[TT];
 #pragma unroll
                     for (int j = 0; j < TT; j++) z[j] = cj(vw[(jb + j)]);
 #pragma unroll
-                    for (int i = 0; i < TT; i++) u[i] = pp[(ib + i)] + al * vw[(ib + i)];
+                    for (int i = 0; i < TT; i++) u[i] = mad(pp[(ib + i)], al, vw[(ib + i)]);
 #pragma unroll
                     for (int i = 0; i < TT; i++)
 #pragma unroll
-                        for (int j = 0; j < TT; j++) A[i][j] -= u[i] * z[j];
+                        for (int j = 0; j < TT; j++) A[i][j] = msub(A[i][j], u[i], z[j]);
                 }
             }
         }
@@ -2192,29 +2269,12 @@ __global__ void __launch_bounds__(TILE_MAX_THREADS, WPE) tridiag_tile_cplx_kerne
         __syncthreads(); /* (3) next column */
     }
     }
-    if (tid == 0) dd[N - 1] = ((N & 1) ? xk0 : xk1)[tvi(N - 1)].x; /* column N-1 was written at step N-2 */
-    __syncthreads();
-    for (int i = tid; i < N; i += blockDim.x) {
-        a.dS[(size_t)i * a.nmat + mat] = dd[i];
-        a.eS[(size_t)i * a.nmat + mat] = (i + 1 < N) ? ee[i] : 0.0;
-        if (a.tauv) reinterpret_cast<zd *>(a.tauv)[(size_t)mat * N + i] = (i + 1 < N) ? tt[i] : zd{0.0, 0.0};
-    }
     if (tid == 0) {
-        double gl = dd[0], gu = dd[0], emax2 = 0.0;
-        for (int i = 0; i < N; i++) {
-            const double di = dd[i];
-            double off = (i > 0 ? fabs(ee[i - 1]) : 0.0) + (i + 1 < N ? fabs(ee[i]) : 0.0);
-            gl = fmin(gl, di - off);
-            gu = fmax(gu, di + off);
-            if (i + 1 < N) emax2 = fmax(emax2, ee[i] * ee[i]);
-        }
-        double tnorm = fmax(fabs(gl), fabs(gu));
-        gl -= 2.0 * DBL_EPSILON * tnorm * N + 1e-300;
-        gu += 2.0 * DBL_EPSILON * tnorm * N + 1e-300;
-        a.gb[4 * mat] = gl;
-        a.gb[4 * mat + 1] = gu;
-        a.gb[4 * mat + 2] = DBL_MIN * fmax(1.0, emax2);
-        a.gb[4 * mat + 3] = tnorm;
+        const double dn = ((N & 1) ? xk0 : xk1)[tvi(N - 1)].x; /* column N-1 was written at step N-2 */
+        a.dS[(size_t)(N - 1) * a.nmat + mat] = dn;
+        a.eS[(size_t)(N - 1) * a.nmat + mat] = 0.0;
+        if (a.tauv) reinterpret_cast<zd *>(a.tauv)[(size_t)mat * N + N - 1] = zd{0.0, 0.0};
+        last_bounds(a, N, mat, bnd, dn);
     }
 }
 
@@ -3731,9 +3791,9 @@ int tridiag_generic(pmx_ctx *c, EigArgs &a, bool real, bool lds_matrix, int grid
         auto tiles = [&](int tt) {
             const int nb_ = (N + tt - 1) / tt;
             const int thr = (std::max(nb_ * (nb_ + 1) / 2, nb_ * tt) + 63) / 64 * 64;
-            const size_t ts = tt + 1;
-            const size_t lds_t = sizeof(zd) * ((3 + thr / 64) * (size_t)nb_ * ts + (size_t)nb_ * (nb_ | 1) * ts + N) +
-                                 sizeof(double) * 2 * (size_t)N;
+            const size_t ts = tt | 1;
+            const size_t lds_t = sizeof(zd) * ((2 + thr / 64) * ((size_t)nb_ * ts + 1) + (size_t)nb_ * (nb_ | 1) * ts) +
+                                 sizeof(double) * 4;
             return std::make_tuple(nb_, thr, lds_t);
         };
         auto add = [&](const char *name, int tt, auto kern) {
@@ -3750,14 +3810,14 @@ int tridiag_generic(pmx_ctx *c, EigArgs &a, bool real, bool lds_matrix, int grid
                                  return 0;
                              }});
         };
-        add("ctile6", 6, tridiag_tile_cplx_kernel<6, 2>);
+        add("ctile6", 6, N <= 126 ? tridiag_tile_cplx_kernel<6, 2, 2> : tridiag_tile_cplx_kernel<6, 3, 2>);
         /* the default, for batches too small to time and untimed runs: register
          * tiles hide none of a step's barriers below five of them.  A call of
-         * bands for 64 matrices, three_stream / fused / ctile6: N 15 114 / 108 /
-         * 119 us, N 30 217 / 207 / 208, N 51 413 / 382 / 273, N 89 1034 / 952 /
-         * 462, N 130 2113 / 1915 / 697 */
+         * bands for 64 matrices, three_stream / fused / ctile6: N 18 120 / 114 /
+         * 126 us, N 30 205 / 192 / 173, N 54 454 / 423 / 256, N 102 1330 / 1214 /
+         * 448, N 130 2097 / 1900 / 599 */
         if (lds_matrix) {
-            const char *pref = N >= 30 ? "ctile6" : "fused";
+            const char *pref = N >= 24 ? "ctile6" : "fused";
             for (size_t i = 1; i < cands.size(); i++)
                 if (std::strcmp(cands[i].name, pref) == 0) std::swap(cands[0], cands[i]);
         }
