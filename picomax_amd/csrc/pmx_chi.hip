@@ -4426,11 +4426,19 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
     if (nk == 0 || nq == 0) return PMX_OK;
     const size_t lds_t = sizeof(double) * 4 * (size_t)nch * D;
     if (lds_t > c->lds_max) return set_error(PMX_EINVAL, "NEPS too large for the adjoint");
-    /* k-points go in batches of at most 512 whose two full eigenvector sets
-     * (at k and at k+q, 16 N^2 bytes per k-point each) stay near 4 GB: the
-     * gradient is a sum over k, so each batch recomputes its eigenpairs and
-     * adds its share, and device memory does not grow with the grid */
-    const int KB = (int)std::max<size_t>(16, std::min<size_t>(512, (size_t)4e9 / (32 * (size_t)N * N + 1)));
+    /* k-points go in batches of at most 2048 whose two full eigenvector sets
+     * (at k and at k+q, 16 N^2 bytes per k-point each) stay near 4 GB, and so
+     * do the overlaps and their gradients beyond 512: the gradient is a sum
+     * over k, so each batch recomputes its eigenpairs and adds its share, and
+     * device memory does not grow with the grid.  512 k-points are two matrices
+     * per CU, where five of order 89 fit: a fit step of GaAs on 12^3 k takes
+     * 20.9 ms in batches of 512 and 16.0 in one */
+    size_t kb = std::max<size_t>(16, std::min<size_t>(2048, (size_t)4e9 / (32 * (size_t)N * N + 1)));
+    if (kb > 512) {
+        const size_t nst = soc ? p->nband : p->nband / 2;
+        kb = std::max<size_t>(512, std::min(kb, (size_t)4e9 / (8 * nst * nst * nch * D + 1))); /* nc nv <= nst^2 / 4 */
+    }
+    const int KB = (int)std::min<size_t>(kb, nk);
 
     /* inverse loci: invl[m][l] = p with loci[m][p] = l (G_p -> G_p + G_m is one to one) */
     std::vector<int> invl((size_t)neps * npw, -1);
