@@ -166,6 +166,7 @@ struct Prof {
     Prof(pmx_ctx *ctx, const char *name, double flops = 0.0, double bytes = 0.0);
     ~Prof();
 };
+bool eig_in_slab(const pmx_ctx *ctx);
 /* eigensolve of nmat H(K) on the context's stream; K is a device array.
  * Eigenvalues of the lowest nb states; eigenvectors of the lowest nvec, or,
  * with vsel = 1 / 2, only of those above / at or below voff (the others are

@@ -1060,10 +1060,61 @@ __global__ void __launch_bounds__(EIG_THREADS, 2) tridiag_panel_kernel(EigArgs a
  *     their use, and the next column and its row of V, W are at hand when the
  *     step begins.
  * N = 582, 61 matrices: 53.5 -> 20.4 ms (288 of N = 401: 30.0 -> 20 ms, where
- * the memory system is the bound: 4.7 TB/s of reads). What is left at N = 582 is
- * half mat-vec (32k cycles a step of loads, 11k of arithmetic beside them) and
- * a quarter panel update. */
+ * the memory system is the bound: 4.7 TB/s of reads). Of a step's 36 us at N =
+ * 582 the mat-vec takes 21 and the panel update 9.7, both bound by what one CU
+ * can load; the row passes and barriers take 5.
+ *
+ * The first two divide over CUs.  With LG > 0, 1 << LG workgroups share a matrix:
+ * each holds and updates its own columns (16 at a time, in turn, in a slab of its
+ * own), and all run the row passes alike on the same bits.  A step exchanges one
+ * vector, the workgroups' shares of A22 v, summed in their order by everyone; a
+ * panel, its columns.  61 matrices of N = 582, four workgroups each: 20.5 -> 11.0
+ * ms, a step 36 -> 19 us, of which about 3 for the exchange. */
 constexpr int WD_THREADS = 512, WD_WAVES = 8, WD_NBP = 4, WD_MR = 2;
+
+/* The columns of one of the 1 << lg workgroups that share a matrix: groups of 16
+ * dealt in turn, workgroup gi's l-th being group (l << lg) + gi. */
+struct WideShare {
+    int gi, lg;
+    __device__ __forceinline__ int group(int l) const { return (l << lg) + gi; }
+    /* how many of its groups lie below group x */
+    __device__ __forceinline__ int below(int x) const { return x > gi ? (x - gi + (1 << lg) - 1) >> lg : 0; }
+    __device__ __forceinline__ bool owns(int c) const { return (((c >> 4) ^ gi) & ((1 << lg) - 1)) == 0; }
+};
+
+/* Entries that other workgroups of the matrix read: stores go through to where
+ * every CU sees them, loads do not take a line this CU or XCD holds. */
+template <class T> __device__ __forceinline__ void xstore(T *p, T v) {
+    double *q = reinterpret_cast<double *>(p);
+    __hip_atomic_store(q, re(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (sizeof(T) == sizeof(zd)) __hip_atomic_store(q + 1, im(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T> __device__ __forceinline__ T xload(const T *p) {
+    const double *q = reinterpret_cast<const double *>(p);
+    const double x = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return mk<T>(x, sizeof(T) == sizeof(zd) ? __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0);
+}
+
+/* what a workgroup publishes lies behind its V and W in its slab: 2 N partial
+ * sums of p (even and odd steps), 4 N entries of the next panel's columns, then a
+ * line with its tick, and in the first slab the launch's ticket counter */
+template <class T> __host__ __device__ __forceinline__ size_t wide_pub_offset(int N) {
+    const size_t P = (size_t)N * (N + 1) / 2;
+    return (P * sizeof(T) + 255) / 256 * 256 + 2 * WD_NBP * (size_t)N * sizeof(T);
+}
+template <class T> __host__ __device__ __forceinline__ size_t wide_tick_offset(int N) {
+    return (wide_pub_offset<T>(N) + (2 + WD_NBP) * (size_t)N * sizeof(T) + 127) / 128 * 128;
+}
+
+/* ticks and the ticket counter to zero before a shared launch */
+__global__ void __launch_bounds__(256) wide_zero_kernel(char *scratch, size_t slab, size_t off, int nwg) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < nwg) {
+        int *t = reinterpret_cast<int *>(scratch + (size_t)i * slab + off);
+        t[0] = 0;
+        t[1] = 0;
+    }
+}
 
 /* tridiag_wide_kernel's trailing update: rows and columns c0..N-1 of the
  * packed lower A, panel columns 0..nb-1 of V and W (the rest count as zero).
@@ -1072,26 +1123,31 @@ constexpr int WD_THREADS = 512, WD_WAVES = 8, WD_NBP = 4, WD_MR = 2;
  * real part and (-W.y, W.x, -V.y, V.x) for the imaginary; real: two panel
  * columns per step, (V, W) against (W, V). */
 template <class T>
-__device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int N, int c0, int nb, int lane, int wave) {
+__device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int N, int c0, int nb, int lane, int wave,
+                                            const WideShare &sh) {
     constexpr bool CX = sizeof(T) == sizeof(zd);
     constexpr int KS = CX ? WD_NBP : WD_NBP / 2; /* K steps */
     typedef double dv4 __attribute__((ext_vector_type(4)));
-    const int L = N - c0;
-    if (L <= 0) return;
-    const int nrb = (L + 63) >> 6, ncg = (L + 15) >> 4;
+    if (c0 >= N) return;
+    const int nrb = (N + 63) >> 6, ncg = (N + 15) >> 4, l0 = sh.below(c0 >> 4);
     asm volatile("" : "+v"(lane)); /* no address hoisted into the caller's loops */
     const int kq = lane >> 4, lc = lane & 15;
     struct Item {
         int rb, cg;
     };
-    /* items row block by row block: column groups 0 .. min(4 rb + 4, ncg) - 1 */
+    /* items row block by row block: this workgroup's column groups from c0's
+     * to min(4 rb + 4, ncg) - 1, counted from 0; what reaches below c0 is
+     * loaded and not stored */
     auto settle = [&](Item it) {
-        while (it.rb < nrb && it.cg >= min(4 * it.rb + 4, ncg)) {
-            it.cg -= min(4 * it.rb + 4, ncg);
+        while (it.rb < nrb) {
+            const int n = sh.below(min(4 * it.rb + 4, ncg)) - l0;
+            if (it.cg < n) break;
+            it.cg -= n;
             it.rb++;
         }
         return it;
     };
+    auto col0 = [&](int cg) { return 16 * sh.group(l0 + cg); };
     /* the panel entry of row or column x that K index kq of step s takes;
      * swap: V and W exchanged (columns), flip: x and y exchanged (imaginary part) */
     auto panel = [&](int s, int x, bool swap, bool flip) -> double {
@@ -1101,30 +1157,31 @@ __device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int 
         const double v = CX ? q[(kq & 1) ^ (flip ? 1 : 0)] : q[0];
         return i < nb ? v : 0.0;
     };
-    Item it = settle(Item{0, wave});
+    Item it = settle(Item{c0 >> 6, wave});
     T cur[4][4], nxt[4][4];       /* [row tile][accumulator]: row 16 t + lc, column kq + 4 v */
     double rf[KS][4];             /* row entries of the current row block */
     double cr[KS], ci[KS];        /* column entries of the current item */
     double nr[KS], ni[KS];        /* and of the next */
     auto load = [&](Item q, T (&b)[4][4], double (&er)[KS], double (&ei)[KS]) {
-        if (q.rb >= nrb) q = Item{0, 0}; /* past the last item: loaded and not used */
+        /* past the last item: row 0 and column 0 loaded and not used */
+        const int cc = q.rb < nrb ? col0(q.cg) : 0, rr = q.rb < nrb ? 64 * q.rb : 0;
 #pragma unroll
         for (int s = 0; s < KS; s++) {
-            er[s] = panel(s, c0 + 16 * q.cg + lc, true, false);
-            ei[s] = CX ? panel(s, c0 + 16 * q.cg + lc, true, true) : 0.0;
+            er[s] = panel(s, cc + lc, true, false);
+            ei[s] = CX ? panel(s, cc + lc, true, true) : 0.0;
         }
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-            const int c = min(c0 + 16 * q.cg + kq + 4 * v, N - 1);
+            const int c = min(cc + kq + 4 * v, N - 1);
             const T *col = A + ((long)pk(c, c, N) - c);
 #pragma unroll
-            for (int t = 0; t < 4; t++) b[t][v] = col[max(min(c0 + 64 * q.rb + 16 * t + lc, N - 1), c)];
+            for (int t = 0; t < 4; t++) b[t][v] = col[max(min(rr + 16 * t + lc, N - 1), c)];
         }
     };
     load(it, cur, cr, ci);
     int have = -1; /* row block in rf */
     while (it.rb < nrb) {
-        const int r0 = c0 + 64 * it.rb, cc = c0 + 16 * it.cg;
+        const int r0 = 64 * it.rb, cc = col0(it.cg);
         if (have != it.rb) {
             have = it.rb;
 #pragma unroll
@@ -1156,7 +1213,7 @@ __device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int 
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int c = cc + kq + 4 * v;
-                if (c < N && r >= c && r < N) A[pk(r, c, N)] = mk<T>(xr[v], CX ? xi[v] : 0.0);
+                if (c >= c0 && c < N && r >= c && r < N) A[pk(r, c, N)] = mk<T>(xr[v], CX ? xi[v] : 0.0);
             }
         }
 #pragma unroll
@@ -1172,8 +1229,10 @@ __device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int 
     }
 }
 
-template <class T>
-__global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) {
+template <class T, int LG>
+__global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, int mat0, int mat1) {
+    constexpr bool SHARED = LG > 0;
+    constexpr int NW = 1 << LG; /* workgroups per matrix */
     extern __shared__ double smem_d[];
     constexpr int NBP = WD_NBP;
     const int N = a.N;
@@ -1193,18 +1252,76 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
     __shared__ T sh_cw[NBP], sh_cv[NBP];   /* conj of row k of W and V */
     __shared__ T sh_cWv[NBP], sh_cVv[NBP]; /* W^H v, V^H v */
 
-    char *slab = a.scratch + (size_t)blockIdx.x * a.slab;
+    /* shared matrices: workgroups take tickets as they start, so those of one
+     * matrix follow each other and none waits for one behind it that its own
+     * place keeps from starting (at most one matrix of a launch is incomplete) */
+    __shared__ int sh_ticket;
+    int wg = blockIdx.x;
+    if (SHARED) {
+        if (tid0 == 0)
+            sh_ticket = __hip_atomic_fetch_add(reinterpret_cast<int *>(a.scratch + wide_tick_offset<T>(N)) + 1, 1,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        wg = __builtin_amdgcn_readfirstlane(sh_ticket);
+    }
+    const WideShare sh{wg & (SHARED ? NW - 1 : 0), LG};
+    char *slab = a.scratch + (size_t)wg * a.slab;
     T *A = reinterpret_cast<T *>(slab);
     T *Vp = reinterpret_cast<T *>(slab + ((P * sizeof(T) + 255) / 256) * 256);
     T *Wp = Vp + (size_t)NBP * N;
+    T *X = reinterpret_cast<T *>(slab + wide_pub_offset<T>(N)), *Cn = X + 2 * (size_t)N;
+    char *slab0 = a.scratch + (size_t)(wg - sh.gi) * a.slab; /* of the matrix's first workgroup */
+    const size_t xoff = wide_pub_offset<T>(N), toff = wide_tick_offset<T>(N);
+    __shared__ int sh_lost;
+    if (SHARED && tid0 == 0) sh_lost = 0; /* before the first meet's barrier */
+    int tick = 0;
+    bool lost = false;
+    /* all published so far is seen by the matrix's other workgroups, and theirs by
+     * this one: a publication has reached memory (sc1 stores, vmcnt 0) before the
+     * tick that announces it is stored.  The wait ends after some seconds whatever happens: the matrix
+     * then gets NaN and nobody waits for it again. */
+    auto meet = [&]() {
+        tick++;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        int *mine = reinterpret_cast<int *>(slab + toff);
+        if (tid0 == 0) __hip_atomic_store(mine, tick, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int *theirs = reinterpret_cast<const int *>(slab0 + (size_t)(lane & (NW - 1)) * a.slab + toff);
+        for (int n = 0; !lost; n++) {
+            const int t = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__all(t >= tick)) break;
+            if (n > (1 << 23)) {
+                lost = true;
+                sh_lost = 1;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        asm volatile("" ::: "memory");
+    };
+    /* the next panel's columns, by their owner */
+    auto publish = [&](int c0) {
+        if (sh.owns(c0))
+            for (int c = c0; c < min(c0 + NBP, N); c++)
+                for (int r = max(c0, c) + tid; r < N; r += WD_THREADS) xstore(Cn + (size_t)(c - c0) * N + r, A[pk(r, c, N)]);
+        meet();
+    };
+    /* row r of column k, stale by j panel columns */
+    auto column = [&](int r, int k, int j) -> T {
+        if (!SHARED) return A[pk(r, k, N)];
+        const char *own = slab0 + (size_t)(((k - j) >> 4) & (NW - 1)) * a.slab;
+        return xload(reinterpret_cast<const T *>(own + xoff) + (size_t)(2 + j) * N + r);
+    };
 
-    for (int mat = blockIdx.x; mat < a.nmat; mat += gridDim.x) {
+    const int mstep = SHARED ? mat1 : gridDim.x; /* a shared launch: one matrix per workgroup */
+    for (int mat = mat0 + (wg >> LG); mat < mat1; mat += mstep) {
         const double Kv[3] = {a.K[3 * mat], a.K[3 * mat + 1], a.K[3 * mat + 2]};
         T *vref = a.vref ? reinterpret_cast<T *>(a.vref) + (size_t)mat * P : nullptr;
         T *tau_out = a.tauv ? reinterpret_cast<T *>(a.tauv) + (size_t)mat * N : nullptr;
         for (int c = wave; c < N; c += WD_WAVES)
-            for (int r = c + lane; r < N; r += 64) A[pk(r, c, N)] = h_elem<T>(a, Kv, r, c);
+            if (!SHARED || sh.owns(c))
+                for (int r = c + lane; r < N; r += 64) A[pk(r, c, N)] = h_elem<T>(a, Kv, r, c);
         __syncthreads();
+        if (SHARED) publish(0);
 
         for (int k0 = 0; k0 + 1 < N; k0 += NBP) {
             const int nb = min(NBP, N - 1 - k0);
@@ -1213,12 +1330,12 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
 #pragma unroll
             for (int m = 0; m < WD_MR; m++) {
                 const int r = tid + WD_THREADS * m;
-                xa[m] = (r >= k0 && r < N) ? A[pk(r, k0, N)] : zero<T>();
+                xa[m] = (r >= k0 && r < N) ? column(r, k0, 0) : zero<T>();
 #pragma unroll
                 for (int i = 0; i < NBP; i++) vi[m][i] = wi[m][i] = zero<T>();
             }
             for (int j = 0; j < nb; j++) {
-                const int k = k0 + j, L = N - k - 1;
+                const int k = k0 + j, R0 = k + 1;
                 /* addresses are formed anew in every step: hoisted out of the loop
                  * they would spill, and a reload inside the mat-vec would wait for
                  * its loads ahead */
@@ -1271,55 +1388,61 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                     if (r >= k + 1 && r < N) {
                         vv[r] = v;
                         Vp[(size_t)j * N + r] = v;
-                        if (vref && r >= k + 2) vref[pk(r, k, N)] = v;
+                        if (vref && r >= k + 2 && (!SHARED || (k & (NW - 1)) == sh.gi)) vref[pk(r, k, N)] = v;
                     }
                 }
                 if (tid == 0) {
                     e[k] = beta;
                     sh_tau = tau;
-                    if (tau_out) tau_out[k] = tau;
+                    if (tau_out && sh.gi == 0) tau_out[k] = tau;
                 }
                 __syncthreads(); /* (2) */
-                /* (c) stale A22 v, every stored element read once.  Local
-                 * column ct and row rr are k + 1 + ct, k + 1 + rr.  A work item
-                 * is four neighbouring columns (quad qd) by two blocks of 64
-                 * rows (group g); a wave takes the quads wave + 8 i that reach
-                 * the group, group by group, and loads two items ahead. */
+                /* (c) stale A22 v, every stored element of this workgroup's columns
+                 * read once.  A work item is four neighbouring columns (quad) by
+                 * two blocks of 64 rows (group g), both counted from row 0; a wave
+                 * takes every eighth quad of the workgroup's (the l-th is l & 3 of
+                 * column group l >> 2) that reaches the group, group by group, and
+                 * loads two items ahead. */
                 {
-                    const T *vk1 = vv + k + 1;
-                    const int nquad = (L + 3) >> 2, ngrp = (L + 127) >> 7;
-                    int g = wave < nquad ? 0 : ngrp, qd = wave; /* fewer quads than waves: none */
-                    int gl = g, ql = qd;                        /* the item to load next */
-                    auto step = [&](int &g, int &qd) {
-                        qd += WD_WAVES;
-                        if (qd >= min(nquad, 32 * (g + 1))) {
+                    const int nquad = (N + 3) >> 2, ngrp = (N + 127) >> 7;
+                    auto quad = [&](int l) { return 4 * sh.group(l >> 2) + (l & 3); };
+                    const int q1 = R0 >> 2, lc1 = sh.below(q1 >> 2);
+                    const int l1 = 4 * lc1 + (sh.group(lc1) == q1 >> 2 ? q1 & 3 : 0); /* the first quad past column k */
+                    const int l0 = l1 + ((wave - l1) & (WD_WAVES - 1));
+                    int g = R0 >> 7;
+                    while (g < ngrp && quad(l0) >= min(nquad, 32 * (g + 1))) g++;
+                    int ql = l0, gl = g, lq = l0; /* this item; the item to load next */
+                    const int gs = g;             /* ngrp: this wave has no part of the product */
+                    auto step = [&](int &g, int &l) {
+                        l += WD_WAVES;
+                        if (quad(l) >= min(nquad, 32 * (g + 1))) {
                             g++;
-                            qd = wave;
+                            l = l0;
                         }
                     };
                     /* every item issues the same eight loads, so the wait before
                      * an item counts only its own.  Rows past the end read row
-                     * L - 1 (their v is 0 and their partials are not stored),
+                     * N - 1 (their v is 0 and their partials are not stored),
                      * rows above the quad read its first row (masked below),
                      * columns past the end read the last one (v 0, dot not
                      * stored); past the last item row 0 of column 0 is loaded
                      * and not used. */
                     auto load = [&](T (&b)[2][4]) {
-                        const int q0 = gl < ngrp ? 4 * ql : 0, c0 = k + 1 + q0, nc = L - q0;
+                        const int c0 = gl < ngrp ? 4 * quad(lq) : 0, nc = N - c0;
                         const int rb = gl < ngrp ? 128 * gl : -128;
-                        const unsigned base = pk(c0, c0, N) - q0;
+                        const unsigned base = pk(c0, c0, N) - c0;
                         const unsigned d1 = nc > 1 ? N - 1 - c0 : 0, d2 = nc > 2 ? d1 + N - 2 - c0 : d1,
                                        d3 = nc > 3 ? d2 + N - 3 - c0 : d2;
                         const unsigned off[4] = {base, base + d1, base + d2, base + d3};
 #pragma unroll
                         for (int h = 0; h < 2; h++) {
-                            const unsigned r = max(min(rb + 64 * h + lane, L - 1), q0);
+                            const unsigned r = max(min(rb + 64 * h + lane, N - 1), c0);
 #pragma unroll
                             for (int t = 0; t < 4; t++)
                                 b[h][t] = *reinterpret_cast<const T *>(reinterpret_cast<const char *>(A) +
                                                                        (unsigned)sizeof(T) * (r + off[t]));
                         }
-                        if (gl < ngrp) step(gl, ql);
+                        if (gl < ngrp) step(gl, lq);
                     };
                     T pt[2], vr[2];
                     auto open_group = [&]() {
@@ -1327,21 +1450,21 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                         for (int h = 0; h < 2; h++) {
                             const int rr = 128 * g + 64 * h + lane;
                             pt[h] = zero<T>();
-                            vr[h] = rr < L ? vk1[min(rr, L - 1)] : zero<T>();
+                            vr[h] = rr >= R0 && rr < N ? vv[min(rr, N - 1)] : zero<T>();
                         }
                     };
                     auto compute = [&](const T (&b)[2][4]) {
-                        const int q0 = 4 * qd;
+                        const int q0 = 4 * quad(ql);
                         T dot[4], vc[4];
 #pragma unroll
                         for (int t = 0; t < 4; t++) {
                             dot[t] = zero<T>();
-                            vc[t] = vk1[min(q0 + t, L - 1)];
+                            vc[t] = vv[min(q0 + t, N - 1)];
                         }
-                        if (q0 + 3 >= L) /* columns past the end */
+                        if (q0 + 3 >= N || q0 < R0) /* columns past the end or before the trailing matrix */
 #pragma unroll
-                            for (int t = 1; t < 4; t++)
-                                if (q0 + t >= L) vc[t] = zero<T>();
+                            for (int t = 0; t < 4; t++)
+                                if (q0 + t >= N || q0 + t < R0) vc[t] = zero<T>();
 #pragma unroll
                         for (int h = 0; h < 2; h++) {
                             const int rb = 128 * g + 64 * h;
@@ -1365,7 +1488,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                                               re(dot[2]), im(dot[2]), re(dot[3]), im(dot[3])};
                         const double tot = wave_sum8(v8, lane);
                         const int wid = wave_sum8_id(lane), ct = q0 + (wid >> 1);
-                        if ((lane & 7) == 0 && ct < L && (sizeof(T) == sizeof(zd) || !(wid & 1))) {
+                        if ((lane & 7) == 0 && ct < N && (sizeof(T) == sizeof(zd) || !(wid & 1))) {
                             double *o = reinterpret_cast<double *>(dotv + ct) + (wid & 1);
                             *o = (q0 >> 7) == g ? tot : *o + tot; /* the column's first group sets it */
                         }
@@ -1379,12 +1502,12 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                         load(fetch);
                         compute(cur);
                         const int g0 = g;
-                        step(g, qd);
+                        step(g, ql);
                         if (g != g0) {
 #pragma unroll
                             for (int h = 0; h < 2; h++) {
                                 const int rr = 128 * g0 + 64 * h + lane;
-                                if (rr < L) part[wave * N + rr] = pt[h];
+                                if (rr < N) part[wave * N + rr] = pt[h];
                             }
                             open_group();
                         }
@@ -1393,15 +1516,15 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                     if (g < ngrp)
                         while (turn(b0, b2) && turn(b1, b0) && turn(b2, b1)) {
                         }
-                    else /* this wave has no part of the product */
-                        for (int rr = lane; rr < L; rr += 64) part[wave * N + rr] = zero<T>();
+                    /* rows above this wave's first item */
+                    for (int rr = R0 + lane; rr < min(128 * gs, N); rr += 64) part[wave * N + rr] = zero<T>();
                     /* W^H v and V^H v: wave i takes column i of the panel */
                     if (wave < j) {
                         T tw = zero<T>(), tv = zero<T>();
-                        for (int rr = lane; rr < L; rr += 64) {
-                            const T w = Wp[(size_t)wave * N + k + 1 + rr], v = Vp[(size_t)wave * N + k + 1 + rr];
-                            tw = madc(tw, w, vk1[rr]);
-                            tv = madc(tv, v, vk1[rr]);
+                        for (int rr = R0 + lane; rr < N; rr += 64) {
+                            const T w = Wp[(size_t)wave * N + rr], v = Vp[(size_t)wave * N + rr];
+                            tw = madc(tw, w, vv[rr]);
+                            tv = madc(tv, v, vv[rr]);
                         }
                         const double v8[8] = {re(tw), im(tw), re(tv), im(tv), 0.0, 0.0, 0.0, 0.0};
                         const double tot = wave_sum8(v8, lane);
@@ -1424,6 +1547,33 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                     }
                 }
                 __syncthreads(); /* (3) */
+                T px[WD_MR]; /* shared: the product's rows */
+                if (SHARED) { /* this workgroup's share out; all shares in, summed in their order */
+#pragma unroll
+                    for (int m = 0; m < WD_MR; m++) {
+                        const int r = tid + WD_THREADS * m;
+                        if (r >= R0 && r < N) {
+                            T p = sh.owns(r) ? dotv[r] : zero<T>();
+#pragma unroll
+                            for (int w = 0; w < WD_WAVES; w++) p += part[w * N + r];
+                            xstore(X + (size_t)(k & 1) * N + r, sh_lost ? from_real<T>(__builtin_nan("")) : p);
+                        }
+                    }
+                    meet();
+                    T q[WD_MR][NW];
+#pragma unroll
+                    for (int m = 0; m < WD_MR; m++)
+#pragma unroll
+                        for (int i = 0; i < NW; i++)
+                            q[m][i] = xload(reinterpret_cast<const T *>(slab0 + (size_t)i * a.slab + xoff) +
+                                            (size_t)(k & 1) * N + min(max(tid + WD_THREADS * m, R0), N - 1));
+#pragma unroll
+                    for (int m = 0; m < WD_MR; m++) {
+                        px[m] = q[m][0];
+#pragma unroll
+                        for (int i = 1; i < NW; i++) px[m] += q[m][i];
+                    }
+                }
                 /* p with the panel's corrections; w = p - (tau/2)(p^H v) v */
                 T ps[WD_MR], vs[WD_MR];
                 double pr = 0.0, pim = 0.0;
@@ -1433,11 +1583,14 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
                     T p = zero<T>();
                     vs[m] = zero<T>();
                     if (r >= k + 1 && r < N) {
-                        const int rr = r - k - 1;
-                        p = dotv[rr];
                         vs[m] = vv[r];
+                        if (SHARED) {
+                            p = px[m];
+                        } else {
+                            p = dotv[r];
 #pragma unroll
-                        for (int w = 0; w < WD_WAVES; w++) p += part[w * N + rr];
+                            for (int w = 0; w < WD_WAVES; w++) p += part[w * N + r];
+                        }
 #pragma unroll
                         for (int i = 0; i < NBP; i++)
                             if (i < j) p = msub(msub(p, vi[m][i], sh_cWv[i]), wi[m][i], sh_cVv[i]);
@@ -1458,7 +1611,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
 #pragma unroll
                 for (int m = 0; m < WD_MR; m++) {
                     const int r = tid + WD_THREADS * m;
-                    xa[m] = (j + 1 < nb && r >= k + 1 && r < N) ? A[pk(r, k + 1, N)] : zero<T>();
+                    xa[m] = (j + 1 < nb && r >= k + 1 && r < N) ? column(r, k + 1, j + 1) : zero<T>();
                 }
                 __syncthreads(); /* (4) */
                 double sr = 0.0, si = 0.0;
@@ -1496,11 +1649,13 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a) 
              * four columns and each load covers 256 contiguous bytes.  A work
              * item is 64 rows by 16 columns, the next one's entries loaded
              * ahead; V and W come straight from the slab. */
-            wide_update<T>(A, Vp, Wp, N, k0 + nb, nb, lane, wave);
+            wide_update<T>(A, Vp, Wp, N, k0 + nb, nb, lane, wave, sh);
             __syncthreads();
+            if (SHARED) publish(k0 + nb);
         }
+        if (SHARED && sh.gi != 0) return; /* its outputs are the first workgroup's to write */
         if (tid == 0) {
-            d[N - 1] = re(A[pk(N - 1, N - 1, N)]);
+            d[N - 1] = SHARED && sh_lost ? __builtin_nan("") : re(column(N - 1, N - 1, 0));
             e[N - 1] = 0.0;
             if (tau_out) tau_out[N - 1] = zero<T>();
         }
@@ -3588,16 +3743,33 @@ size_t lds_wide_bytes(int N, size_t elem) {
     return elem * (2 + WD_WAVES) * (size_t)N + sizeof(double) * 2 * (size_t)N;
 }
 
-/* one matrix per CU (bases whose vectors and partials fit the LDS) */
+/* One matrix per CU (bases whose vectors and partials fit the LDS); matrices
+ * that would leave half of the CUs idle, a small batch or the rest of a larger
+ * one, are shared by 2, 4 or 8 workgroups, as many as there are CUs for.  A call
+ * of bands in ms, 1 / 2 / 4 / 8 workgroups: 8 matrices of N = 218 2.68 / 2.54 /
+ * 2.28 / 2.28, of 610 20.8 / 14.6 / 10.3 / 8.6; 61 of 610 21.3 / 15.2 / 11.7 (no
+ * room for 8); 121 of 610 25.7 / 19.9; 300 of 610, 44 of them shared, 69.4 / 56.2
+ * / 52.1. */
 template <class T> int launch_tridiag_wide(pmx_ctx *c, EigArgs &a, int grid, size_t lds) {
-    auto go = [&](auto kern) -> int {
+    auto go = [&](auto kern, int g, int mat0, int mat1) -> int {
         if (lds > 65536)
             PMX_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(WD_THREADS), lds, c->stream, a);
+        hipLaunchKernelGGL(kern, dim3(g), dim3(WD_THREADS), lds, c->stream, a, mat0, mat1);
         PMX_CHECK_HIP(hipGetLastError());
         return 0;
     };
-    return go(tridiag_wide_kernel<T>);
+    const int rest = a.nmat % c->num_cu, full = a.nmat - rest;
+    const size_t toff = wide_tick_offset<T>(a.N), slabs = c->dScratch.n * sizeof(double) / a.slab;
+    int lg = 0;
+    while (rest > 0 && lg < 3 && (rest << (lg + 1)) <= c->num_cu && (size_t)(rest << (lg + 1)) <= slabs) lg++;
+    if (lg == 0 || a.slab < toff + 2 * sizeof(int)) return go(tridiag_wide_kernel<T, 0>, grid, 0, a.nmat);
+    int rc;
+    if (full > 0 && (rc = go(tridiag_wide_kernel<T, 0>, std::min(grid, full), 0, full))) return rc;
+    const int nwg = rest << lg;
+    hipLaunchKernelGGL(wide_zero_kernel, dim3((nwg + 255) / 256), dim3(256), 0, c->stream, a.scratch, a.slab, toff, nwg);
+    PMX_CHECK_HIP(hipGetLastError());
+    return go(lg == 1 ? tridiag_wide_kernel<T, 1> : lg == 2 ? tridiag_wide_kernel<T, 2> : tridiag_wide_kernel<T, 3>, nwg, full,
+              a.nmat);
 }
 
 /* Lanes per eigenvalue: as many as keep the batch within two waves on every
@@ -3926,6 +4098,11 @@ template <class T> int launch_backtrans(pmx_ctx *c, int N, int nmat, int nvec, c
 }
 
 } // namespace
+
+/* whether the system's matrices lie in global memory during the tridiagonalisation */
+bool eig_in_slab(const pmx_ctx *c) {
+    return lds_bytes(basis_size(c), !c->soc && c->real_gauge ? sizeof(double) : sizeof(zd), true) > c->lds_max;
+}
 
 static int eig_device_run(pmx_ctx *c, int nmat, const double *dKpts, int nb, int nvec, double *dEvals, zd *dEvecs,
                           int vsel, double voff, int nsplit, int vsel2) {

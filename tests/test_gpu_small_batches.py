@@ -133,3 +133,24 @@ def test_vectors_of_small_complex_bases(gcut2, us, nk):
         assert np.abs(ev[k] - np.linalg.eigvalsh(H)[:nb]).max() < 1e-10
         assert np.abs(H @ V - V * ev[k]).max() < 1e-9
     ctx.close()
+
+
+# large bases shared by 2, 4 and 8 workgroups, and the rest of a batch that fills
+# the GPU once; last panels of 1 to 4 columns, one and two rows a thread
+@pytest.mark.parametrize("args,gcut2,nk", [(TE, 9.6, 128), (TE, 16.0, 64), (TE + TE_SO, 9.0, 33), (TE + TE_SO, 16.0, 100),
+                                           (TE + TE_SO, 16.0, 40), (TE, 10.6, 257), (SI, 36.0, 90), (SI, 48.0, 60),
+                                           (SI, 80.0, 7)])
+def test_shared_large_bases(args, gcut2, nk):
+    """Eigenvalues against one matrix per call (1e-10 eV), which the test above holds to numpy; orthonormal vectors."""
+    ctx = capi.Context(0)
+    inp = capi.Input(args + ["-gcut", repr(gcut2 ** 0.5)])
+    ctx.set_system(inp.system(), inp)
+    K = np.random.default_rng(nk).uniform(-0.4, 0.4, (nk, 3))
+    ev, vec = ctx.eig(K, 20, vectors=True)
+    for k in range(0, nk, max(1, nk // 5)):
+        one, _ = ctx.eig(K[k:k + 1], 20, vectors=True)
+        assert np.abs(ev[k] - one[0]).max() < 1e-10
+    for k in (0, nk - 1):
+        z = vec[k]
+        assert np.abs(z.conj() @ z.T - np.eye(len(z))).max() < 1e-10
+    ctx.close()
