@@ -2992,6 +2992,27 @@ __global__ void qnext_kernel(int *qstate) {
  * to process end, one copy per GPU, so that entry point calls no allocator.
  * Host code never uses this name as an address (on the host it is a stand-in
  * symbol); it uses the per-device pointer from hipGetSymbolAddress below. */
+/* the eigenpairs of the current q of a batch (slot q % nqb) to the slot that a
+ * captured step reads */
+__global__ void __launch_bounds__(256) qslot_kernel(const int *qstate, int nqb, size_t nev, size_t nvk, const double *ev,
+                                                    const zd *vk, double *ev_to, zd *vk_to) {
+    const size_t slot = qstate[0] % nqb, t0 = (size_t)blockIdx.x * 256 + threadIdx.x, nt = (size_t)gridDim.x * 256;
+    for (size_t i = t0; i < nev; i += nt) ev_to[i] = ev[slot * nev + i];
+    for (size_t i = t0; i < nvk; i += nt) vk_to[i] = vk[slot * nvk + i];
+}
+
+/* q values whose k+q points are solved in one batch with those at k.  A basis
+ * whose matrix lies in global memory takes a CU to itself, and a batch takes as
+ * long for one matrix as for one per CU, so few k-points are batched over q, up
+ * to the two per CU below which no kernels are timed, and 4 GB of eigenvectors.
+ * Spin-orbit Te, 48 k, 3 q, N = 582: batches of 96, 48 and 48 took 62.4 ms to
+ * tridiagonalise, one of 192 takes 22. */
+int q_batch(const pmx_ctx *c, int nk, int nq, size_t bytes_per_k) {
+    if (!eig_in_slab(c)) return 1;
+    const size_t n = std::min((size_t)(2 * c->num_cu - 1) / nk, ((size_t)4 << 30) / (bytes_per_k * nk));
+    return (int)std::max<size_t>(1, std::min<size_t>(nq, n > 1 ? n - 1 : 1));
+}
+
 constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)32 << 20;
 static __device__ __align__(256) zd scratch[NOALLOC_SCRATCH_BYTES / sizeof(zd)];
 
@@ -3175,24 +3196,40 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
     head("  Solving for |k,v>...");
 
     /* ---- phase A: eigenpairs at k (src/pmx_chi.cpp:379-413), solved in one
-     * batch with those at k+q of the first q: [K; K + Q_0].  Eigenpairs at k
-     * fill the first half of evk/vk, those at k+q the second. */
+     * batch with those at k+q of the first nqb q: [K; K + Q_0; ...].
+     * Eigenpairs at k fill slot 0 of evk/vk, those at k+q of q slot
+     * 1 + q % nqb; with nqb > 1 a captured step reads a slot of its own. */
+    const int nqb = q_batch(c, p->nk, p->nq, (size_t)nb_s * N * sizeof(zd));
     std::vector<double> Kh(p->K, p->K + 3 * p->nk);
     std::vector<double> KWh(p->KW, p->KW + p->nk);
     std::vector<double> K2(Kh);
-    if (p->nq > 0)
+    for (int q = 0; q < (nqb > 1 ? p->nq : std::min(p->nq, 1)); q++)
         for (int k = 0; k < p->nk; k++)
-            for (int d = 0; d < 3; d++) K2.push_back(Kh[3 * k + d] + p->Q[d]);
+            for (int d = 0; d < 3; d++) K2.push_back(Kh[3 * k + d] + p->Q[3 * q + d]);
     if ((rc = upload(st, w.Kd, K2)) || (rc = upload(st, w.KWd, KWh))) return rc;
-    if ((rc = w.evk.ensure((size_t)2 * p->nk * nb_s)) || (rc = w.vk.ensure((size_t)2 * p->nk * nb_s * N))) return rc;
-    double *evk_p = w.evk.p, *evkq_p = w.evk.p + (size_t)p->nk * nb_s;
-    zd *vk_p = w.vk.p, *vkq_p = w.vk.p + (size_t)p->nk * nb_s * N;
+    const size_t ev_slot = (size_t)p->nk * nb_s, vk_slot = ev_slot * N;
+    const int nslot = nqb > 1 ? nqb + 2 : 2;
+    if ((rc = w.evk.ensure(nslot * ev_slot)) || (rc = w.vk.ensure(nslot * vk_slot))) return rc;
+    double *evk_p = w.evk.p, *evkq_p = w.evk.p + ev_slot;
+    zd *vk_p = w.vk.p, *vkq_p = w.vk.p + vk_slot;
     /* rho reads bra rows at k (conduction; chi_xyz: valence) and ket rows at
      * k+q (valence; chi_xyz: conduction) only */
     const int vsel_k = xyz ? 2 : 1, vsel_kq = xyz ? 1 : 2;
-    if ((rc = eig_device(c, p->nq > 0 ? 2 * p->nk : p->nk, w.Kd.p, nb_s, nb_s, evk_p, vk_p, vsel_k, p->offset,
+    if ((rc = eig_device(c, (1 + std::min(p->nq, nqb)) * p->nk, w.Kd.p, nb_s, nb_s, evk_p, vk_p, vsel_k, p->offset,
                          p->nk, vsel_kq)))
         return rc;
+    /* nqb > 1: the group of q whose eigenpairs the slots hold, and the solve of
+     * another one (its k+q points follow K in Kd) */
+    int q_have = 0;
+    auto solve_group = [&](int q) -> int {
+        const int q0 = q / nqb * nqb;
+        if (q0 == q_have) return 0;
+        const int n = std::min(nqb, p->nq - q0);
+        const int r = eig_device(c, n * p->nk, w.Kd.p + 3 * (size_t)p->nk * (1 + q0), nb_s, nb_s, w.evk.p + ev_slot,
+                                 w.vk.p + vk_slot, vsel_kq, p->offset);
+        q_have = r ? -1 : q0;
+        return r;
+    };
     if ((rc = elapsed("  "))) return rc;
     head(std::string("  Solving for susceptibility tensor matrix elements") +
          (xyz ? " (xyz-basis)" : ll ? " (alternative form)" : "") + "...");
@@ -3251,11 +3288,16 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
         if (c->progress) std::cout << "  (" << (q + 1) << "/" << p->nq << ")..." << std::endl;
         head("    Solving for overlap integrals...");
         if (cap) {
-            QSelArgs qa{w.qstate.p, neps * 9, neps * 3 * npw, 3 * p->nk, w.ucAll.p, w.wAAll.p,
+            QSelArgs qa{w.qstate.p, neps * 9, neps * 3 * npw, nqb > 1 ? 0 : 3 * p->nk, w.ucAll.p, w.wAAll.p,
                         spatial ? nullptr : w.wSAll.p, w.KQAll.p, w.QAll.p, w.ucd.p, w.wAd.p,
                         spatial ? nullptr : w.wSd.p, w.KQd.p, w.Qcur.p, w.bad.p};
             hipLaunchKernelGGL(qsel_kernel, dim3(256), dim3(256), 0, st, qa);
-            if ((rc = eig_device(c, p->nk, w.KQd.p, nb_s, nb_s, evkq_p, vkq_p, vsel_kq, p->offset))) return rc;
+            if (nqb > 1) {
+                evkq_p = w.evk.p + (nqb + 1) * ev_slot;
+                vkq_p = w.vk.p + (nqb + 1) * vk_slot;
+                hipLaunchKernelGGL(qslot_kernel, dim3(4 * c->num_cu), dim3(256), 0, st, w.qstate.p, nqb, ev_slot, vk_slot,
+                                   w.evk.p + ev_slot, w.vk.p + vk_slot, evkq_p, vkq_p);
+            } else if ((rc = eig_device(c, p->nk, w.KQd.p, nb_s, nb_s, evkq_p, vkq_p, vsel_kq, p->offset))) return rc;
         } else {
             /* ---- per-q tables: uvec_LT (src/pmx_basis.cpp:830-874), weights */
             std::vector<zd> uc, wA, wS;
@@ -3270,7 +3312,11 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
                 KQ[3 * k + 1] = Kh[3 * k + 1] + Qy;
                 KQ[3 * k + 2] = Kh[3 * k + 2] + Qz;
             }
-            if (q > 0) {
+            if (nqb > 1) {
+                if ((rc = solve_group(q))) return rc;
+                evkq_p = w.evk.p + (1 + q % nqb) * ev_slot;
+                vkq_p = w.vk.p + (1 + q % nqb) * vk_slot;
+            } else if (q > 0) {
                 if ((rc = upload(st, w.KQd, KQ))) return rc;
                 if ((rc = eig_device(c, p->nk, w.KQd.p, nb_s, nb_s, evkq_p, vkq_p, vsel_kq, p->offset))) return rc;
             }
@@ -3742,6 +3788,10 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
         if (ok) {
             c->qstep_captures++;
             int qq = q;
+            if (nqb > 1 && (rc = solve_group(qq))) {
+                (void)hipGraphExecDestroy(exec);
+                return rc;
+            }
             PMX_CHECK_HIP(hipGraphLaunch(exec, st));
             c->qstep_replays++;
             qq++;
@@ -3749,6 +3799,11 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
             PMX_CHECK_HIP(hipMemcpyAsync(&first_flag, w.qstate.p + 2 + q, sizeof(int), hipMemcpyDeviceToHost, st));
             PMX_CHECK_HIP(hipStreamSynchronize(st));
             for (; !first_flag && qq < p->nq; qq++) {
+                if (nqb > 1 && (rc = solve_group(qq))) {
+                    (void)hipStreamSynchronize(st);
+                    (void)hipGraphExecDestroy(exec);
+                    return rc;
+                }
                 PMX_CHECK_HIP(hipGraphLaunch(exec, st));
                 c->qstep_replays++;
             }

@@ -154,3 +154,28 @@ def test_shared_large_bases(args, gcut2, nk):
         z = vec[k]
         assert np.abs(z.conj() @ z.T - np.eye(len(z))).max() < 1e-10
     ctx.close()
+
+
+# bases in global memory, q in one batch with k: all at once, in groups (100 k:
+# four q at a time), with and without a captured step, the smallest counts
+@pytest.mark.parametrize("nk,nq", [(1, 2), (3, 3), (8, 7), (100, 3), (100, 4), (100, 6), (100, 9), (170, 2), (171, 3), (260, 2)])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_q_batches(nk, nq, precision):
+    """A list of q against one q per call: the same products in the same order, up to the eigensolver's rounding."""
+    ctx = capi.Context(0)
+    inp = capi.Input(TE + ["-gcut", repr(9.6 ** 0.5), "-neps", "3"])
+    ctx.set_system(inp.system(), inp)
+    K = np.random.default_rng(nk).uniform(-0.4, 0.4, (nk, 3))
+    KW = np.full(nk, 1.0 / nk)
+    Q = np.array([[0.0, 0.0, 0.03 * (i + 1)] for i in range(nq)])
+    e = ctx.bands(np.concatenate([K] + [K + q for q in Q]), 24, 0.0)
+    off = (e[:, 0].max() + e[:, 23].min()) / 2  # states on both sides of it at every point
+    a = (24, off, 1, 0.1, 60, 0.1, 1)
+    for _ in range(2):
+        got = ctx.chi(K, KW, Q, *a, precision=precision)
+        one = [ctx.chi(K, KW, q[None, :], *a, precision=precision) for q in Q]
+        for i in (0, 1):
+            g = got[i].reshape(9, nq, -1)
+            w = np.stack([o[i].reshape(9, -1) for o in one], 1)
+            assert np.abs(g - w).max() < (1e-10 if precision == "fp64" else 1e-5) * np.abs(w).max()
+    ctx.close()
