@@ -47,23 +47,36 @@ class BandModel:
         return self.ctx.ref_energy(self.refpoint, self.nvalence)
 
     def bands(self, K, nband):
-        return self.ctx.bands(K, nband, self.offset())
+        K = np.asarray(K, float).reshape(-1, 3)
+        n, n2 = self.nvalence, 2 * self.sys.npw
+        if not 0 < n <= n2 or nband <= 0 or len(K) == 0:
+            return self.ctx.bands(K, nband, self.offset())
+        # the offset's own solve as one more point of the batch: alone it takes as long as 64 points
+        # (GaAs, 89 plane waves: 0.39 ms)
+        e = self.ctx.bands(np.concatenate([K, self.refpoint[None, :]]), max(int(nband), min(n + 1, n2)), 0.0)
+        off = (e[-1, n - 1] + e[-1, min(n, n2 - 1)]) / 2.0
+        out = e[:-1, :nband] - off
+        out[:, n2:] = 0.0
+        return out
 
     def grad(self, K, nband, gE):
         """sum_{k,n} gE[k,n] d eband[k,n] / d vg (offset term included)."""
         K = np.asarray(K, float).reshape(-1, 3)
         gE = np.asarray(gE, float).reshape(len(K), nband)
-        g = np.zeros((self.natom, self.nv))
-        for k0 in range(0, len(K), self.batch):
-            g += self.ctx.grad_bands(K[k0:k0 + self.batch], nband, gE[k0:k0 + self.batch])
         nvb = self.nvalence
         tot = gE.sum()
         if tot != 0.0 and 0 < nvb < 2 * self.sys.npw:
-            # offset = (E_{nv-1} + E_nv)/2 at the reference point
-            gref = np.zeros((1, nvb + 1))
-            gref[0, nvb - 1] = -0.5 * tot
-            gref[0, nvb] = -0.5 * tot
-            g += self.ctx.grad_bands(self.refpoint[None, :], nvb + 1, gref)
+            # offset = (E_{nv-1} + E_nv)/2 at the reference point, one more point of the last batch
+            # (alone it takes as long as 64 points: GaAs, 89 plane waves, 0.65 ms)
+            ref = np.zeros((1, max(nband, nvb + 1)))
+            ref[0, nvb - 1] = ref[0, nvb] = -0.5 * tot
+            gE = np.concatenate([np.pad(gE, ((0, 0), (0, ref.shape[1] - nband))), ref])
+            K = np.concatenate([K, self.refpoint[None, :]])
+            nband = ref.shape[1]
+        g = np.zeros((self.natom, self.nv))
+        step = self.batch + (len(K) % self.batch == 1 < len(K))
+        for k0 in range(0, len(K), step):
+            g += self.ctx.grad_bands(K[k0:k0 + step], nband, gE[k0:k0 + step])
         return g
 
 
