@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256) rho_kernel(RhoArgs a) {
     const double Kx = a.K[3 * k], Ky = a.K[3 * k + 1], Kz = a.K[3 * k + 2];
     const zd *vk = a.vk + (size_t)k * a.nb_s * a.N;
     const zd *vkq = a.vkq + (size_t)k * a.nb_s * a.N;
-    for (int job = threadIdx.x; job < npair * a.neps; job += blockDim.x) {
+    for (int job = threadIdx.x + 256 * blockIdx.y; job < npair * a.neps; job += 256 * gridDim.y) {
         const int m = job / npair, t = job % npair;
         const int row = a.pos[tb + t];
         if (row < 0) continue;
@@ -328,7 +328,7 @@ template <class T> __global__ void __launch_bounds__(256) rho_mfma_kernel(RhoArg
     const int nvg = (nvs + 3) / 4;            /* valence column groups of 4 */
     const int nct = (ncs + 15) / 16;          /* conduction row tiles */
     const int jobs = a.neps * nct * nvg;
-    for (int job = wave; job < jobs; job += 4) {
+    for (int job = wave + 4 * blockIdx.y; job < jobs; job += 4 * gridDim.y) {
         const int m = job / (nct * nvg), rem = job % (nct * nvg);
         const int ct = rem / nvg, vg = rem % nvg;
         const int crow = ct * 16 + (lane & 15);            /* A row */
@@ -478,7 +478,7 @@ template <class T> __global__ void __launch_bounds__(256, 4) rho_cart_kernel(Rho
     const int ncol = a.neps * nvs;            /* (m, v) columns, v fastest */
     const int nct = (ncs + 15) / 16, njt = (ncol + 15) / 16;
     const int K2 = 2 * a.npw, kq = lane >> 4;
-    for (int job = wave; job < nct * njt; job += 4) {
+    for (int job = wave + 4 * blockIdx.y; job < nct * njt; job += 4 * gridDim.y) {
         const int ct = job / njt, jt = job % njt;
         const int crow = ct * 16 + (lane & 15); /* A row */
         const int col = jt * 16 + (lane & 15);  /* B column */
@@ -618,7 +618,7 @@ __global__ void __launch_bounds__(256, 3) rho_bf3_kernel(RhoArgs a, int K2p) {
     const int ncol = a.neps * nvs; /* (m, v) columns, v fastest */
     const int nct = (ncs + 15) / 16, njt = (ncol + 15) / 16;
     const int kq8 = 8 * (lane >> 4);
-    for (int job = wave; job < nct * njt; job += 4) {
+    for (int job = wave + 4 * blockIdx.y; job < nct * njt; job += 4 * gridDim.y) {
         const int ct = job / njt, jt = job % njt;
         const int crow = ct * 16 + (lane & 15); /* A row */
         const int col = jt * 16 + (lane & 15);  /* B column */
@@ -771,7 +771,7 @@ template <class T> __global__ void __launch_bounds__(256, 2) rho_soc_kernel(RhoA
     const int ncol = a.neps * nvs; /* (m, v) columns, v fastest */
     const int nct = (ncs + 15) / 16, njt = (ncol + 15) / 16;
     const int KP = 2 * a.npw, kq = lane >> 4;
-    for (int job = wave; job < nct * njt; job += 4) {
+    for (int job = wave + 4 * blockIdx.y; job < nct * njt; job += 4 * gridDim.y) {
         const int ct = job / njt, jt = job % njt;
         const int crow = ct * 16 + (lane & 15); /* A row */
         const int col = jt * 16 + (lane & 15);  /* B column */
@@ -3437,9 +3437,12 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
                 PMX_CHECK_HIP(hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_r));
             }
             /* SOC: the valence spinor rows at k+q and the G table */
-            int maxnv = cap ? nv_cap : 0;
+            int maxnc = cap ? nc_cap : 0, maxnv = cap ? nv_cap : 0;
             if (!cap)
-                for (int kk = 0; kk < p->nk; kk++) maxnv = std::max(maxnv, nvh[kk]);
+                for (int kk = 0; kk < p->nk; kk++) {
+                    maxnc = std::max(maxnc, nch_h[kk]);
+                    maxnv = std::max(maxnv, nvh[kk]);
+                }
             const size_t lds_soc = sizeof(float2) * (size_t)maxnv * N + sizeof(float) * 3 * (size_t)npw;
             /* the Cartesian form: its LDS is the rows plus the G table */
             const size_t lds_c = lds_r + (fp32 ? sizeof(float) : sizeof(double)) * 3 * (size_t)npw;
@@ -3453,6 +3456,16 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
                 }
             const int K2p = (2 * npw + 31) & ~31;
             const size_t lds_b = 4 * (size_t)maxnc2 * K2p + sizeof(float2) * (size_t)maxnv2 * N + sizeof(float) * 3 * (size_t)npw;
+            /* few k-points: each one's tiles over several workgroups, as many as
+             * find a place on the GPU at once (each stages the rows of its k
+             * again) and have a tile for every wave.  Spin-orbit Te, 48 k, N =
+             * 582, 43 G: rho_soc_kernel 3.53 -> 0.88 ms a q */
+            auto rho_grid = [&](size_t lds, int jobs, int resident) {
+                const int fit = lds > 0 ? std::max(1, std::min(resident, (int)(c->lds_max / lds))) : resident;
+                const int split = std::min(fit * c->num_cu / p->nk, (jobs + 3) / 4);
+                return dim3(p->nk, std::max(1, split));
+            };
+            auto tiles = [](int n) { return (n + 15) / 16; };
             const char *rf = std::getenv("PMX_RHO");
             const bool rho_bf = spatial && fp32 && p->precision == PMX_PREC_BF16X3 && N == npw &&
                                 lds_b <= c->lds_max && !(rf && std::strcmp(rf, "fp32") == 0);
@@ -3460,23 +3473,23 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
                 if (lds_b > 65536)
                     PMX_CHECK_HIP(hipFuncSetAttribute((const void *)rho_bf3_kernel,
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_b));
-                hipLaunchKernelGGL(rho_bf3_kernel, dim3(p->nk), dim3(256), lds_b, st, ra, K2p);
+                hipLaunchKernelGGL(rho_bf3_kernel, rho_grid(lds_b, tiles(maxnc2) * tiles(neps * maxnv2), 3), dim3(256), lds_b, st, ra, K2p);
             } else if (rho_lds && fp32 && lds_c <= c->lds_max) {
                 if (lds_c > 65536)
                     PMX_CHECK_HIP(hipFuncSetAttribute((const void *)rho_cart_kernel<float>,
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_c));
-                hipLaunchKernelGGL(rho_cart_kernel<float>, dim3(p->nk), dim3(256), lds_c, st, ra);
+                hipLaunchKernelGGL(rho_cart_kernel<float>, rho_grid(lds_c, tiles(maxnc2) * tiles(neps * maxnv2), 4), dim3(256), lds_c, st, ra);
             } else if (rho_lds && fp32)
-                hipLaunchKernelGGL(rho_mfma_kernel<float>, dim3(p->nk), dim3(256), lds_r, st, ra);
+                hipLaunchKernelGGL(rho_mfma_kernel<float>, rho_grid(lds_r, neps * tiles(maxnc2) * ((maxnv2 + 3) / 4), 4), dim3(256), lds_r, st, ra);
             else if (rho_lds)
-                hipLaunchKernelGGL(rho_mfma_kernel<double>, dim3(p->nk), dim3(256), lds_r, st, ra);
+                hipLaunchKernelGGL(rho_mfma_kernel<double>, rho_grid(lds_r, neps * tiles(maxnc2) * ((maxnv2 + 3) / 4), 4), dim3(256), lds_r, st, ra);
             else if (!spatial && !ll && fp32 && lds_soc <= c->lds_max) {
                 if (lds_soc > 65536)
                     PMX_CHECK_HIP(hipFuncSetAttribute((const void *)rho_soc_kernel<float>,
                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_soc));
-                hipLaunchKernelGGL(rho_soc_kernel<float>, dim3(p->nk), dim3(256), lds_soc, st, ra);
+                hipLaunchKernelGGL(rho_soc_kernel<float>, rho_grid(lds_soc, tiles(maxnc) * tiles(neps * maxnv), 2), dim3(256), lds_soc, st, ra);
             } else
-                hipLaunchKernelGGL(rho_kernel, dim3(p->nk), dim3(256), 0, st, ra);
+                hipLaunchKernelGGL(rho_kernel, rho_grid(0, (maxnc * maxnv * neps + 63) / 64, 8), dim3(256), 0, st, ra);
         }
         PMX_CHECK_HIP(hipGetLastError());
         if ((rc = elapsed("    "))) return rc;
