@@ -4248,7 +4248,18 @@ __device__ __forceinline__ void spin_grads(const zd *gx, int D, int col, zd &gup
     gdu = zd{gB.x - gE.x, gB.y - gE.y};
 }
 
-/* step (4): one block per k (it owns row k of every output) */
+/* c + a b and c + conj(a) b as chains of FMAs */
+__device__ __forceinline__ zd cmad(zd c, zd a, zd b) {
+    return zd{fma(-a.y, b.y, fma(a.x, b.x, c.x)), fma(a.y, b.x, fma(a.x, b.y, c.y))};
+}
+__device__ __forceinline__ zd cmadc(zd c, zd a, zd b) {
+    return zd{fma(a.y, b.y, fma(a.x, b.x, c.x)), fma(-a.y, b.x, fma(a.x, b.y, c.y))};
+}
+
+/* step (4): one block per k (it owns row k of every output).  Bound by its loads
+ * and FP64 products: per m the weights are loaded once for all partner states and
+ * the three directions meet before the state they multiply.  1,728 k, N = 89, 9 G:
+ * 1.10 ms with the partner states outermost, now 0.45 ms. */
 __global__ void __launch_bounds__(256) chi_adj_evec_kernel(AdjVArgs a) {
     const int k = blockIdx.x;
     const int ncs = a.soc ? a.nc[k] : a.nc[k] / 2, nvs = a.soc ? a.nv[k] : a.nv[k] / 2;
@@ -4270,30 +4281,40 @@ __global__ void __launch_bounds__(256) chi_adj_evec_kernel(AdjVArgs a) {
         const int c = idx / a.npw, p = idx % a.npw;
         const int cst = nst - 1 - c;
         zd su{0, 0}, sd{0, 0};
-        for (int v = 0; v < nvs; v++) {
-            const zd *gx = a.gX + (tb + (size_t)c * nvs + v) * CD;
-            const zd *cq = vkq + (size_t)v * a.N;
-            for (int m = 0; m < a.neps; m++) {
-                const int l = a.loci[(size_t)m * a.npw + p];
-                if (l < 0) continue;
-                for (int i = 0; i < 3; i++) {
-                    const int col = 3 * m + i;
-                    const zd wa = a.wA[((size_t)m * 3 + i) * a.npw + p], b = bk[col];
-                    const zd W{wa.x + b.x, wa.y + b.y};
-                    if (!a.soc) {
-                        const zd r = cmul(cconj(gx[col]), cmul(cq[l], W));
-                        su.x += r.x; su.y += r.y;
-                    } else {
+        const zd *gc = a.gX + (tb + (size_t)c * nvs) * CD;
+        for (int m = 0; m < a.neps; m++) {
+            const int l = a.loci[(size_t)m * a.npw + p];
+            if (l < 0) continue;
+            zd W[3], S[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const zd wa = a.wA[((size_t)m * 3 + i) * a.npw + p], b = bk[3 * m + i];
+                W[i] = zd{wa.x + b.x, wa.y + b.y};
+                if (a.soc) S[i] = a.wS[((size_t)m * 3 + i) * a.npw + p];
+            }
+            for (int v = 0; v < nvs; v++) {
+                const zd *gx = gc + (size_t)v * CD;
+                const zd *cq = vkq + (size_t)v * a.N;
+                if (!a.soc) {
+                    zd t{0, 0};
+#pragma unroll
+                    for (int i = 0; i < 3; i++) t = cmadc(t, gx[3 * m + i], W[i]);
+                    su = cmad(su, t, cq[l]);
+                } else {
+                    /* up bra: rho_up (W, up ket), rho_ud (S, down ket); down bra: rho_dn, rho_du */
+                    zd t1{0, 0}, t2{0, 0}, t3{0, 0}, t4{0, 0};
+#pragma unroll
+                    for (int i = 0; i < 3; i++) {
                         zd gup, gdn, gud, gdu;
-                        spin_grads(gx, a.D, col, gup, gdn, gud, gdu);
-                        const zd S = a.wS[((size_t)m * 3 + i) * a.npw + p];
-                        const zd qu = cq[2 * l], qd = cq[2 * l + 1];
-                        /* up bra: rho_up (W, up ket), rho_ud (S, down ket); down bra: rho_dn, rho_du */
-                        const zd r1 = cmul(cconj(gup), cmul(qu, W)), r2 = cmul(cconj(gud), cmul(qd, S));
-                        const zd r3 = cmul(cconj(gdn), cmul(qd, W)), r4 = cmul(cconj(gdu), cmul(qu, S));
-                        su.x += r1.x + r2.x; su.y += r1.y + r2.y;
-                        sd.x += r3.x + r4.x; sd.y += r3.y + r4.y;
+                        spin_grads(gx, a.D, 3 * m + i, gup, gdn, gud, gdu);
+                        t1 = cmadc(t1, gup, W[i]);
+                        t2 = cmadc(t2, gud, S[i]);
+                        t3 = cmadc(t3, gdn, W[i]);
+                        t4 = cmadc(t4, gdu, S[i]);
                     }
+                    const zd qu = cq[2 * l], qd = cq[2 * l + 1];
+                    su = cmad(cmad(su, t1, qu), t2, qd);
+                    sd = cmad(cmad(sd, t3, qd), t4, qu);
                 }
             }
         }
@@ -4309,32 +4330,39 @@ __global__ void __launch_bounds__(256) chi_adj_evec_kernel(AdjVArgs a) {
     for (int idx = threadIdx.x; idx < nvs * a.npw; idx += 256) {
         const int v = idx / a.npw, l = idx % a.npw;
         zd su{0, 0}, sd{0, 0};
-        for (int c = 0; c < ncs; c++) {
-            const int cst = nst - 1 - c;
-            const zd *gx = a.gX + (tb + (size_t)c * nvs + v) * CD;
-            const zd *ck = vk + (size_t)cst * a.N;
-            for (int m = 0; m < a.neps; m++) {
-                const int p = a.invl[(size_t)m * a.npw + l];
-                if (p < 0) continue;
-                for (int i = 0; i < 3; i++) {
-                    const int col = 3 * m + i;
-                    const zd wa = a.wA[((size_t)m * 3 + i) * a.npw + p], b = bk[col];
-                    const zd Wc{wa.x + b.x, -(wa.y + b.y)};
-                    if (!a.soc) {
-                        const zd r = cmul(gx[col], cmul(ck[p], Wc));
-                        su.x += r.x; su.y += r.y;
-                    } else {
+        for (int m = 0; m < a.neps; m++) {
+            const int p = a.invl[(size_t)m * a.npw + l];
+            if (p < 0) continue;
+            zd W[3], S[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                const zd wa = a.wA[((size_t)m * 3 + i) * a.npw + p], b = bk[3 * m + i];
+                W[i] = zd{wa.x + b.x, wa.y + b.y};
+                if (a.soc) S[i] = a.wS[((size_t)m * 3 + i) * a.npw + p];
+            }
+            for (int c = 0; c < ncs; c++) {
+                const zd *gx = a.gX + (tb + (size_t)c * nvs + v) * CD;
+                const zd *ck = vk + (size_t)(nst - 1 - c) * a.N;
+                if (!a.soc) {
+                    zd t{0, 0};
+#pragma unroll
+                    for (int i = 0; i < 3; i++) t = cmadc(t, W[i], gx[3 * m + i]);
+                    su = cmad(su, t, ck[p]);
+                } else {
+                    /* up ket: rho_up (up bra, W), rho_du (down bra, S); down ket: rho_dn, rho_ud */
+                    zd t1{0, 0}, t2{0, 0}, t3{0, 0}, t4{0, 0};
+#pragma unroll
+                    for (int i = 0; i < 3; i++) {
                         zd gup, gdn, gud, gdu;
-                        spin_grads(gx, a.D, col, gup, gdn, gud, gdu);
-                        const zd Sv = a.wS[((size_t)m * 3 + i) * a.npw + p];
-                        const zd Sc{Sv.x, -Sv.y};
-                        const zd cu = ck[2 * p], cd = ck[2 * p + 1];
-                        /* up ket: rho_up (up bra, W), rho_du (down bra, S); down ket: rho_dn, rho_ud */
-                        const zd r1 = cmul(gup, cmul(cu, Wc)), r2 = cmul(gdu, cmul(cd, Sc));
-                        const zd r3 = cmul(gdn, cmul(cd, Wc)), r4 = cmul(gud, cmul(cu, Sc));
-                        su.x += r1.x + r2.x; su.y += r1.y + r2.y;
-                        sd.x += r3.x + r4.x; sd.y += r3.y + r4.y;
+                        spin_grads(gx, a.D, 3 * m + i, gup, gdn, gud, gdu);
+                        t1 = cmadc(t1, W[i], gup);
+                        t2 = cmadc(t2, S[i], gdu);
+                        t3 = cmadc(t3, W[i], gdn);
+                        t4 = cmadc(t4, S[i], gud);
                     }
+                    const zd cu = ck[2 * p], cd = ck[2 * p + 1];
+                    su = cmad(cmad(su, t1, cu), t2, cd);
+                    sd = cmad(cmad(sd, t3, cd), t4, cu);
                 }
             }
         }
@@ -4358,50 +4386,97 @@ __global__ void __launch_bounds__(256) chi_adj_evec_kernel(AdjVArgs a) {
     }
 }
 
-/* step (5): one block per (k, state n < nbs); psi [nk][N][N] state rows */
-__global__ void __launch_bounds__(256) adj_y_kernel(int N, int nbs, double tol, const zd *psi, const double *ev,
+/* step (5): y_n = sum_m P_m <P_m|g_n> / (E_n - E_m) over the whole basis: two
+ * products with the states P [N][N] of a k on FP64 MFMA, for 16 n at a time, the
+ * coefficients of mc states m between them in LDS.  With one block per (k, n)
+ * each read the states twice, the first time a row per thread: 1.39 ms at 1,728 k,
+ * N = 89, 18 n, at k and at k+q together; now 0.59 ms (3.9 GFLOP).  Blocks: k by
+ * groups of 16 n. */
+constexpr int ADJY_MC = 224; /* states per chunk: 61 KB of coefficients */
+constexpr int ADJY_RS = 17;  /* LDS row of a state's 16 coefficients (bank spread) */
+__global__ void __launch_bounds__(256) adj_y_kernel(int N, int nbs, int mc, double tol, const zd *psi, const double *ev,
                                                     const zd *g, const double *gE, zd *y, int *live) {
-    const int k = blockIdx.x / nbs, n = blockIdx.x % nbs;
+    const int nt = (nbs + 15) / 16, k = blockIdx.x / nt, n0 = blockIdx.x % nt * 16;
     extern __shared__ double ysm[];
-    zd *coef = reinterpret_cast<zd *>(ysm); /* [N] */
+    zd *coef = reinterpret_cast<zd *>(ysm); /* [mc][ADJY_RS] */
+    __shared__ int any[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lc = lane & 15, kq = lane >> 4;
     const zd *P = psi + (size_t)k * N * N;
-    const zd *gn = g + ((size_t)k * nbs + n) * N;
-    const double En = ev[(size_t)k * N + n], gEn = gE[(size_t)k * nbs + n];
-    int nz = gEn != 0.0;
-    for (int p = threadIdx.x; p < N; p += 256) nz |= (gn[p].x != 0.0 || gn[p].y != 0.0);
-    nz = __syncthreads_or(nz);
-    if (!nz) {
-        if (threadIdx.x == 0) live[blockIdx.x] = 0;
-        return;
-    }
-    for (int m = threadIdx.x; m < N; m += 256) {
-        zd cf{0, 0};
-        if (m == n) {
-            cf.x = gEn;
-        } else {
-            const double d = En - ev[(size_t)k * N + m];
-            if (fabs(d) > tol) {
-                zd s{0, 0};
-                const zd *pm = P + (size_t)m * N;
-                for (int p = 0; p < N; p++) {
-                    const zd r = cmul(cconj(pm[p]), gn[p]);
-                    s.x += r.x; s.y += r.y;
-                }
-                cf = zd{s.x / d, s.y / d};
-            }
+    const double *evn = ev + (size_t)k * N;
+    const size_t kn0 = (size_t)k * nbs + n0;
+    for (int r = 4 * wave; r < 4 * wave + 4; r++) {
+        bool nz = false;
+        if (n0 + r < nbs) {
+            nz = gE[kn0 + r] != 0.0;
+            const zd *gn = g + (kn0 + r) * N;
+            for (int p = lane; p < N; p += 64) nz |= gn[p].x != 0.0 || gn[p].y != 0.0;
         }
-        coef[m] = cf;
+        const int on = __any(nz) != 0;
+        if (lane == 0) {
+            any[r] = on;
+            if (n0 + r < nbs) live[kn0 + r] = on;
+        }
     }
     __syncthreads();
-    for (int p = threadIdx.x; p < N; p += 256) {
-        zd s{0, 0};
-        for (int m = 0; m < N; m++) {
-            const zd r = cmul(P[(size_t)m * N + p], coef[m]);
-            s.x += r.x; s.y += r.y;
+    int some = 0;
+#pragma unroll
+    for (int r = 0; r < 16; r++) some |= any[r];
+    if (!some) return;
+    const bool row_ok = n0 + lc < nbs;
+    const zd *ga = g + (kn0 + (row_ok ? lc : 0)) * N;
+    for (int mb = 0; mb < N; mb += mc) {
+        const int me = min(mc, N - mb);
+        for (int mt = 16 * wave; mt < me; mt += 64) {
+            const int m = mb + mt + lc;
+            const zd *pm = P + (size_t)min(m, N - 1) * N;
+            dx4 cr = {0, 0, 0, 0}, ci = {0, 0, 0, 0};
+#pragma unroll 4
+            for (int p0 = 0; p0 < N; p0 += 4) {
+                const int pc = min(p0 + kq, N - 1);
+                zd a = ga[pc], b = pm[pc];
+                if (p0 + kq >= N || !row_ok) a = zd{0, 0};
+                cr = RhoT<double>::mma(a.x, b.x, cr);
+                ci = RhoT<double>::mma(a.y, b.x, ci);
+                cr = RhoT<double>::mma(a.y, b.y, cr);
+                ci = RhoT<double>::mma(-a.x, b.y, ci);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = RhoT<double>::drow(lane, v), n = n0 + r;
+                zd cf{0, 0};
+                if (mt + lc < me && n < nbs) {
+                    const double d = evn[n] - evn[m];
+                    if (m == n) cf.x = gE[kn0 + r];
+                    else if (fabs(d) > tol) cf = zd{cr[v] / d, ci[v] / d};
+                }
+                coef[(mt + lc) * ADJY_RS + r] = cf;
+            }
         }
-        y[((size_t)k * nbs + n) * N + p] = s;
+        __syncthreads();
+        for (int pt = 16 * wave; pt < N; pt += 64) {
+            const int p = pt + lc, pc = min(p, N - 1);
+            dx4 yr = {0, 0, 0, 0}, yi = {0, 0, 0, 0};
+#pragma unroll 4
+            for (int m0 = 0; m0 < me; m0 += 4) { /* coefficients past me are zero up to its tile */
+                const zd cf = coef[(m0 + kq) * ADJY_RS + lc];
+                const zd b = P[(size_t)min(mb + m0 + kq, N - 1) * N + pc];
+                yr = RhoT<double>::mma(cf.x, b.x, yr);
+                yi = RhoT<double>::mma(cf.y, b.x, yi);
+                yr = RhoT<double>::mma(-cf.y, b.y, yr);
+                yi = RhoT<double>::mma(cf.x, b.y, yi);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = RhoT<double>::drow(lane, v);
+                if (p < N && n0 + r < nbs && any[r]) {
+                    zd &o = y[(kn0 + r) * N + p];
+                    const zd t{yr[v], yi[v]};
+                    o = mb > 0 ? zd{o.x + t.x, o.y + t.y} : t;
+                }
+            }
+        }
+        __syncthreads();
     }
-    if (threadIdx.x == 0) live[blockIdx.x] = 1;
 }
 
 /* step (6): one block per (k, n); the adjoint form of hf_grad_kernel */
@@ -4560,7 +4635,8 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
         if ((rc = upload(st, KkT, kt)) || (rc = gr0.ensure((size_t)nel * nfreq)) || (rc = gi0.ensure((size_t)nel * nfreq)))
             return rc;
     }
-    const size_t lds_y = sizeof(zd) * (size_t)N;
+    const int mc_y = std::min((N + 15) / 16 * 16, ADJY_MC), nt_y = (nbs + 15) / 16;
+    const size_t lds_y = sizeof(zd) * ADJY_RS * (size_t)mc_y;
     const size_t lds_hf = sizeof(double) * c->natom * c->nv;
     const unsigned ggrid = (unsigned)std::min<size_t>(((size_t)nel * nfreq + 255) / 256, 8192);
     for (int k0 = 0; k0 < nk; k0 += KB) {
@@ -4644,7 +4720,7 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
                         invd.p, wAd.p, ucd.p, soc ? wSd.p : nullptr, Kd.p, gX.p, gdE.p, gk.p, gkq.p, gEk.p, gEkq.p};
             hipLaunchKernelGGL(chi_adj_evec_kernel, dim3(nkb), dim3(256), sizeof(zd) * 3 * neps, st, av);
             /* (5)-(6) for the states at k+q */
-            hipLaunchKernelGGL(adj_y_kernel, dim3(nkb * nbs), dim3(256), lds_y, st, N, nbs, tol, vkq.p, evkq.p, gkq.p,
+            hipLaunchKernelGGL(adj_y_kernel, dim3(nkb * nt_y), dim3(256), lds_y, st, N, nbs, mc_y, tol, vkq.p, evkq.p, gkq.p,
                                gEkq.p, Y.p, live.p);
             hipLaunchKernelGGL(hf_adj_kernel, dim3(nkb * nbs), dim3(256), lds_hf, st, npw, N, c->natom, c->nv, nbs,
                                soc ? 1 : 0, vkq.p, Y.p, live.p, c->dShell.p, c->dSfac.p, out.p);
@@ -4653,7 +4729,7 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
             PMX_CHECK_HIP(hipStreamSynchronize(st));
         }
         /* (5)-(6) for the states at k of this batch, accumulated over q */
-        hipLaunchKernelGGL(adj_y_kernel, dim3(nkb * nbs), dim3(256), lds_y, st, N, nbs, tol, vk.p, evk.p, gk.p, gEk.p,
+        hipLaunchKernelGGL(adj_y_kernel, dim3(nkb * nt_y), dim3(256), lds_y, st, N, nbs, mc_y, tol, vk.p, evk.p, gk.p, gEk.p,
                            Y.p, live.p);
         hipLaunchKernelGGL(hf_adj_kernel, dim3(nkb * nbs), dim3(256), lds_hf, st, npw, N, c->natom, c->nv, nbs,
                            soc ? 1 : 0, vk.p, Y.p, live.p, c->dShell.p, c->dSfac.p, out.p);

@@ -179,3 +179,33 @@ def test_q_batches(nk, nq, precision):
             w = np.stack([o[i].reshape(9, -1) for o in one], 1)
             assert np.abs(g - w).max() < (1e-10 if precision == "fp64" else 1e-5) * np.abs(w).max()
     ctx.close()
+
+
+# bases below, at and above 16 states a tile, and one of two chunks of states (N > 224)
+@pytest.mark.parametrize("args,gcut2,nband", [(SI, 3.1, 12), (SI, 8.1, 20), (SI, 12.0, 34), (TE, 13.6, 20), (TE + TE_SO, 9.0, 20)])
+def test_chi_gradient_over_bases(args, gcut2, nband):
+    """Directional derivative of a chi functional against central differences: h = 1e-5 Ry, truncation and
+    rounding together below 1e-5 of the gradient's scale."""
+    ctx = capi.Context(0)
+    inp = capi.Input(args + ["-gcut", repr(gcut2 ** 0.5), "-neps", "2"])
+    sysm = inp.system()
+    ctx.set_system(sysm, inp)
+    v0 = np.ctypeslib.as_array(sysm.vg, shape=(sysm.natom, sysm.nv)).copy()
+    K = np.array([[0.11, 0.07, 0.19], [0.23, -0.05, 0.31]])
+    Q = [[0.02, 0.01, 0.03]]
+    e = ctx.bands(np.concatenate([K, K + Q[0]]), nband, 0.0)
+    n = 2 * (np.argmax((e[:, 2::2].min(0) - e[:, 1:-2:2].max(0))) + 1)
+    off = (e[:, n].min() + e[:, n - 1].max()) / 2
+    a = (K, [0.5, 0.5], Q, nband, off, 1, 0.5, 40, 0.25)
+    r = np.random.default_rng(3)
+    re, im = ctx.chi(*a, kk=1)
+    gr, gi = r.normal(size=re.shape), r.normal(size=im.shape)
+    g = ctx.grad_chi(*a, gr, gi, kk=1)
+    dv, h = r.normal(size=v0.shape), 1e-5
+    f = []
+    for sgn in (1, -1):
+        ctx.set_form_factors(v0 + sgn * h * dv)
+        x, y = ctx.chi(*a, kk=1)
+        f.append((gr * x + gi * y).sum())
+    ctx.close()
+    assert abs((f[0] - f[1]) / (2 * h) - (g * dv).sum()) < 1e-5 * np.abs(g * dv).sum()
