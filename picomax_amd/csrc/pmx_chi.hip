@@ -3006,7 +3006,7 @@ __global__ void __launch_bounds__(256) qslot_kernel(const int *qstate, int nqb, 
  * long for one matrix as for one per CU, so few k-points are batched over q, up
  * to the two per CU below which no kernels are timed, and 4 GB of eigenvectors.
  * Spin-orbit Te, 48 k, 3 q, N = 582: batches of 96, 48 and 48 took 62.4 ms to
- * tridiagonalise, one of 192 takes 22. */
+ * tridiagonalise, one of 192 takes 32. */
 int q_batch(const pmx_ctx *c, int nk, int nq, size_t bytes_per_k) {
     if (!eig_in_slab(c)) return 1;
     const size_t n = std::min((size_t)(2 * c->num_cu - 1) / nk, ((size_t)4 << 30) / (bytes_per_k * nk));
