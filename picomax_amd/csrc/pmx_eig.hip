@@ -1278,7 +1278,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
     bool lost = false;
     /* all published so far is seen by the matrix's other workgroups, and theirs by
      * this one: a publication has reached memory (sc1 stores, vmcnt 0) before the
-     * tick that announces it is stored.  The wait ends after some seconds whatever happens: the matrix
+     * tick that announces it is stored.  The wait ends after half a minute whatever happens: the matrix
      * then gets NaN and nobody waits for it again. */
     auto meet = [&]() {
         tick++;
@@ -1290,7 +1290,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
         for (int n = 0; !lost; n++) {
             const int t = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (__all(t >= tick)) break;
-            if (n > (1 << 23)) {
+            if (n > (1 << 25)) {
                 lost = true;
                 sh_lost = 1;
             }
