@@ -2892,7 +2892,18 @@ template <class T> int upload(hipStream_t s, DBuf<T> &b, const std::vector<T> &h
 
 } // namespace
 
+/* the buffers of the adjoint of chi: kept with the context, grown to the largest
+ * call (at most 4 GB of eigenvectors at k and as much at k+q) and freed with it.
+ * Allocated and freed by each call they cost 2.2 ms of a fit step of GaAs on 12^3 k
+ * (14.2 -> 12.0 ms). */
+struct AdjWork {
+    DBuf<double> Kd, KQd, KWd, evk, evkq, dEd, wtd, gdE, gEk, gEkq, gr, gi, gr0, gi0, KkT, out, gReD, gImD;
+    DBuf<zd> vk, vkq, X, gX, gk, gkq, Y, ucd, wAd, wSd, gZ;
+    DBuf<int> invd, nc, nv, tbase, pos, bad, act, arow, live;
+};
+
 struct ChiWork {
+    AdjWork adj;
     DBuf<double> Kd, KQd, KWd, evk, dEd, wtd, Ktd, Kkd, Re0, Im0, ReD, ImD; /* evk, vk: [k; k+q] halves */
     DBuf<double> ws, ss, es, qgn;
     DBuf<zd> vk, Xd, M1, M2, Z1, Z2, Zp, wAd, ucd, wSd; /* Zp: the direct sum's segments */
@@ -4607,9 +4618,9 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
             pairs_q[q].push_back(3 * n + ij % 3);
         }
     const size_t nup = (size_t)nel * nq * nfreq;
-    DBuf<double> Kd, KQd, KWd, evk, evkq, dEd, wtd, gdE, gEk, gEkq, gr, gi, gr0, gi0, KkT, out, gReD, gImD;
-    DBuf<zd> vk, vkq, X, gX, gk, gkq, Y, ucd, wAd, wSd, gZ;
-    DBuf<int> invd, nc, nv, tbase, pos, bad, act, arow, live;
+    if (!c->chi) c->chi = new ChiWork();
+    auto &[Kd, KQd, KWd, evk, evkq, dEd, wtd, gdE, gEk, gEkq, gr, gi, gr0, gi0, KkT, out, gReD, gImD, vk, vkq, X, gX, gk, gkq,
+           Y, ucd, wAd, wSd, gZ, invd, nc, nv, tbase, pos, bad, act, arow, live] = c->chi->adj;
     int rc;
     if ((rc = upload(st, invd, invl)) || (rc = gReD.ensure(nup)) || (rc = gImD.ensure(nup))) return rc;
     PMX_CHECK_HIP(hipMemcpyAsync(gReD.p, gRe, sizeof(double) * nup, hipMemcpyHostToDevice, st));

@@ -29,3 +29,20 @@ def test_offset_in_the_batch(nk, nband, nvalence):
         ref[0, nvalence - 1:] = -0.5 * g.sum()
         want += m.ctx.grad_bands(m.refpoint[None, :], nvalence + 1, ref)
     assert np.abs(m.grad(K, nband, g) - want).max() < 1e-9 * np.abs(want).max()
+
+
+def test_adjoint_buffers_between_calls():
+    """Calls of several sizes on one context, larger and smaller in turn, against a context of their own."""
+    r = np.random.default_rng(1)
+    vary = [(12, 20, 2, 30), (3, 12, 1, 9), (12, 20, 2, 30), (20, 24, 1, 50), (1, 12, 3, 5), (20, 24, 1, 50)]
+    m = autograd.BandModel(ARGS, nvalence=8)
+    for nk, nband, nq, nfreq in vary:
+        K, KW, Q = r.uniform(-0.5, 0.5, (nk, 3)), np.full(nk, 1.0 / nk), r.uniform(0.01, 0.1, (nq, 3))
+        e = m.ctx.bands(np.concatenate([K] + [K + q for q in Q]), nband, 0.0)
+        a = (K, KW, Q, nband, (e[:, 0].max() + e[:, nband - 1].min()) / 2, 1, 0.3, nfreq, 0.2)
+        g, gre, gim = (r.normal(size=n) for n in ((nk, nband), 9 * nq * nfreq, 9 * nq * nfreq))
+        own = autograd.BandModel(ARGS, nvalence=8)
+        for f in (lambda c: c.grad_bands(K, nband, g), lambda c: c.grad_chi(*a, gre, gim, kk=1)):
+            want = f(own.ctx)
+            for _ in range(3):
+                assert np.abs(f(m.ctx) - want).max() < 1e-9 * np.abs(want).max()
