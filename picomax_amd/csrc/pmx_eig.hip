@@ -1097,7 +1097,8 @@ template <class T> __device__ __forceinline__ T xload(const T *p) {
 
 /* what a workgroup publishes lies behind its V and W in its slab: 2 N partial
  * sums of p (even and odd steps), 4 N entries of the next panel's columns, then a
- * line with its tick, and in the first slab the launch's ticket counter */
+ * line [tick, tickets taken, matrix lost, a matrix lost]: the ticket counter and the
+ * last in the launch's first slab, the third in the matrix's first */
 template <class T> __host__ __device__ __forceinline__ size_t wide_pub_offset(int N) {
     const size_t P = (size_t)N * (N + 1) / 2;
     return (P * sizeof(T) + 255) / 256 * 256 + 2 * WD_NBP * (size_t)N * sizeof(T);
@@ -1105,14 +1106,16 @@ template <class T> __host__ __device__ __forceinline__ size_t wide_pub_offset(in
 template <class T> __host__ __device__ __forceinline__ size_t wide_tick_offset(int N) {
     return (wide_pub_offset<T>(N) + (2 + WD_NBP) * (size_t)N * sizeof(T) + 127) / 128 * 128;
 }
+constexpr int WD_LINE = 4; /* ints of a slab's line */
+/* polls of one wait, about a second; a step takes some 20 us */
+constexpr int WD_SPINS = 1 << 20;
 
-/* ticks and the ticket counter to zero before a shared launch */
+/* the lines of a shared launch's slabs to zero before it */
 __global__ void __launch_bounds__(256) wide_zero_kernel(char *scratch, size_t slab, size_t off, int nwg) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < nwg) {
         int *t = reinterpret_cast<int *>(scratch + (size_t)i * slab + off);
-        t[0] = 0;
-        t[1] = 0;
+        for (int j = 0; j < WD_LINE; j++) t[j] = 0;
     }
 }
 
@@ -1229,8 +1232,10 @@ __device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int 
     }
 }
 
-template <class T, int LG>
-__global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, int mat0, int mat1) {
+/* arg: polls of a wait of the shared form before it gives up.  REDO: only the matrices
+ * that a shared launch with 1 << arg workgroups each has marked as lost. */
+template <class T, int LG, bool REDO = false>
+__global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, int mat0, int mat1, int arg) {
     constexpr bool SHARED = LG > 0;
     constexpr int NW = 1 << LG; /* workgroups per matrix */
     extern __shared__ double smem_d[];
@@ -1272,14 +1277,14 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
     T *X = reinterpret_cast<T *>(slab + wide_pub_offset<T>(N)), *Cn = X + 2 * (size_t)N;
     char *slab0 = a.scratch + (size_t)(wg - sh.gi) * a.slab; /* of the matrix's first workgroup */
     const size_t xoff = wide_pub_offset<T>(N), toff = wide_tick_offset<T>(N);
-    __shared__ int sh_lost;
-    if (SHARED && tid0 == 0) sh_lost = 0; /* before the first meet's barrier */
     int tick = 0;
     bool lost = false;
     /* all published so far is seen by the matrix's other workgroups, and theirs by
      * this one: a publication has reached memory (sc1 stores, vmcnt 0) before the
-     * tick that announces it is stored.  The wait ends after half a minute whatever happens: the matrix
-     * then gets NaN and nobody waits for it again. */
+     * tick that announces it is stored.  A wait may end without them: a workgroup that
+     * is not resident (a queue with few CUs) or not scheduled for long sends nothing.
+     * The matrix is then marked, nobody waits long for anyone any more, and the launch
+     * that follows reduces it again, one workgroup by itself. */
     auto meet = [&]() {
         tick++;
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1290,9 +1295,12 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
         for (int n = 0; !lost; n++) {
             const int t = __hip_atomic_load(theirs, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (__all(t >= tick)) break;
-            if (n > (1 << 25)) {
-                lost = true;
-                sh_lost = 1;
+            int *given_up = reinterpret_cast<int *>(a.scratch + toff) + 3;
+            lost = n >= arg ||
+                   ((n & 1023) == 1023 && __hip_atomic_load(given_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if (lost) {
+                __hip_atomic_store(reinterpret_cast<int *>(slab0 + toff) + 2, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(given_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __builtin_amdgcn_s_sleep(1);
         }
@@ -1314,6 +1322,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
 
     const int mstep = SHARED ? mat1 : gridDim.x; /* a shared launch: one matrix per workgroup */
     for (int mat = mat0 + (wg >> LG); mat < mat1; mat += mstep) {
+        if (REDO && !reinterpret_cast<const int *>(a.scratch + ((size_t)(mat - mat0) << arg) * a.slab + toff)[2]) continue;
         const double Kv[3] = {a.K[3 * mat], a.K[3 * mat + 1], a.K[3 * mat + 2]};
         T *vref = a.vref ? reinterpret_cast<T *>(a.vref) + (size_t)mat * P : nullptr;
         T *tau_out = a.tauv ? reinterpret_cast<T *>(a.tauv) + (size_t)mat * N : nullptr;
@@ -1556,7 +1565,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
                             T p = sh.owns(r) ? dotv[r] : zero<T>();
 #pragma unroll
                             for (int w = 0; w < WD_WAVES; w++) p += part[w * N + r];
-                            xstore(X + (size_t)(k & 1) * N + r, sh_lost ? from_real<T>(__builtin_nan("")) : p);
+                            xstore(X + (size_t)(k & 1) * N + r, p);
                         }
                     }
                     meet();
@@ -1655,7 +1664,7 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
         }
         if (SHARED && sh.gi != 0) return; /* its outputs are the first workgroup's to write */
         if (tid == 0) {
-            d[N - 1] = SHARED && sh_lost ? __builtin_nan("") : re(column(N - 1, N - 1, 0));
+            d[N - 1] = re(column(N - 1, N - 1, 0));
             e[N - 1] = 0.0;
             if (tau_out) tau_out[N - 1] = zero<T>();
         }
@@ -3751,10 +3760,12 @@ size_t lds_wide_bytes(int N, size_t elem) {
  * room for 8); 121 of 610 25.7 / 19.9; 300 of 610, 44 of them shared, 69.4 / 56.2
  * / 52.1. */
 template <class T> int launch_tridiag_wide(pmx_ctx *c, EigArgs &a, int grid, size_t lds) {
-    auto go = [&](auto kern, int g, int mat0, int mat1) -> int {
+    const char *se = std::getenv("PMX_WIDE_SPINS");
+    const int spins = se ? std::atoi(se) : WD_SPINS;
+    auto go = [&](auto kern, int g, int mat0, int mat1, int arg) -> int {
         if (lds > 65536)
             PMX_CHECK_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        hipLaunchKernelGGL(kern, dim3(g), dim3(WD_THREADS), lds, c->stream, a, mat0, mat1);
+        hipLaunchKernelGGL(kern, dim3(g), dim3(WD_THREADS), lds, c->stream, a, mat0, mat1, arg);
         PMX_CHECK_HIP(hipGetLastError());
         return 0;
     };
@@ -3762,14 +3773,17 @@ template <class T> int launch_tridiag_wide(pmx_ctx *c, EigArgs &a, int grid, siz
     const size_t toff = wide_tick_offset<T>(a.N), slabs = c->dScratch.n * sizeof(double) / a.slab;
     int lg = 0;
     while (rest > 0 && lg < 3 && (rest << (lg + 1)) <= c->num_cu && (size_t)(rest << (lg + 1)) <= slabs) lg++;
-    if (lg == 0 || a.slab < toff + 2 * sizeof(int)) return go(tridiag_wide_kernel<T, 0>, grid, 0, a.nmat);
+    if (lg == 0 || a.slab < toff + WD_LINE * sizeof(int)) return go(tridiag_wide_kernel<T, 0>, grid, 0, a.nmat, 0);
     int rc;
-    if (full > 0 && (rc = go(tridiag_wide_kernel<T, 0>, std::min(grid, full), 0, full))) return rc;
+    if (full > 0 && (rc = go(tridiag_wide_kernel<T, 0>, std::min(grid, full), 0, full, 0))) return rc;
     const int nwg = rest << lg;
     hipLaunchKernelGGL(wide_zero_kernel, dim3((nwg + 255) / 256), dim3(256), 0, c->stream, a.scratch, a.slab, toff, nwg);
     PMX_CHECK_HIP(hipGetLastError());
-    return go(lg == 1 ? tridiag_wide_kernel<T, 1> : lg == 2 ? tridiag_wide_kernel<T, 2> : tridiag_wide_kernel<T, 3>, nwg, full,
-              a.nmat);
+    if ((rc = go(lg == 1 ? tridiag_wide_kernel<T, 1> : lg == 2 ? tridiag_wide_kernel<T, 2> : tridiag_wide_kernel<T, 3>, nwg,
+                 full, a.nmat, spins)))
+        return rc;
+    /* what a wait has lost, again; nothing to do, it ends at once */
+    return go(tridiag_wide_kernel<T, 0, true>, rest, full, a.nmat, lg);
 }
 
 /* Lanes per eigenvalue: as many as keep the batch within two waves on every
