@@ -1201,12 +1201,11 @@ __device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int 
         }
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            dv4 xr, xi;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                xr[v] = re(cur[t][v]);
-                xi[v] = im(cur[t][v]);
-            }
+            /* the products are summed by themselves, so an entry is rounded at its own
+             * magnitude once a panel: levels of N = 146 to 0.34 eps ||H|| rms, as from
+             * tridiag_panel_kernel; with the entry as accumulator, four roundings a
+             * panel column, 0.47.  The same time (61 of N = 582: 11.7 ms). */
+            dv4 xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0};
 #pragma unroll
             for (int s = 0; s < KS; s++) {
                 xr = __builtin_amdgcn_mfma_f64_16x16x4f64(cr[s], rf[s][t], xr, 0, 0, 0);
@@ -1216,7 +1215,8 @@ __device__ __forceinline__ void wide_update(T *A, const T *Vp, const T *Wp, int 
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int c = cc + kq + 4 * v;
-                if (c >= c0 && c < N && r >= c && r < N) A[pk(r, c, N)] = mk<T>(xr[v], CX ? xi[v] : 0.0);
+                if (c >= c0 && c < N && r >= c && r < N)
+                    A[pk(r, c, N)] = mk<T>(re(cur[t][v]) + xr[v], CX ? im(cur[t][v]) + xi[v] : 0.0);
             }
         }
 #pragma unroll
@@ -1355,10 +1355,11 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
 #pragma unroll
                 for (int m = 0; m < WD_MR; m++) {
                     const int r = tid + WD_THREADS * m;
-                    T x = xa[m];
+                    T t = zero<T>();
 #pragma unroll
                     for (int i = 0; i < NBP; i++)
-                        if (i < j) x = msub(msub(x, vi[m][i], sh_cw[i]), wi[m][i], sh_cv[i]);
+                        if (i < j) t = mad(mad(t, vi[m][i], sh_cw[i]), wi[m][i], sh_cv[i]);
+                    const T x = xa[m] - t;
                     if (r < N) {
                         if (r == k) d[k] = re(x);
                         if (r == k + 1) {
@@ -1600,10 +1601,11 @@ __global__ void __launch_bounds__(WD_THREADS, 2) tridiag_wide_kernel(EigArgs a, 
 #pragma unroll
                             for (int w = 0; w < WD_WAVES; w++) p += part[w * N + r];
                         }
+                        T t = zero<T>();
 #pragma unroll
                         for (int i = 0; i < NBP; i++)
-                            if (i < j) p = msub(msub(p, vi[m][i], sh_cWv[i]), wi[m][i], sh_cVv[i]);
-                        p = sh_tau * p;
+                            if (i < j) t = mad(mad(t, vi[m][i], sh_cWv[i]), wi[m][i], sh_cVv[i]);
+                        p = sh_tau * (p - t);
                         const T cvp = cj(p) * vs[m];
                         pr += re(cvp);
                         pim += im(cvp);
