@@ -2548,11 +2548,12 @@ __global__ void __launch_bounds__(256) bisect_kernel(int N, int nmat, int nb, in
  * j alone (count(lo) = j, count(hi) = j + 1) the probes cut it into L + 1
  * equal parts.  From there lane 0 probes the Newton candidate x - 1/s of the
  * bracket end that is closer by its own step (the midpoint if that falls
- * outside), the others cut the bracket into L parts.  It stops when the
- * bracket or the Newton step is at the rounding level of T: 2 eps |x| + 4
- * pivmin plus a fraction of eps ||T||, below which counts and steps are noise
- * (without that term a level near zero never meets the test).  A level takes
- * about 7 passes with L = 64 and 15 with one thread. */
+ * outside), the others cut the bracket into L parts.  It stops where
+ * bisect_kernel does, 2 eps |x| + 4 pivmin, so that a level far below ||T|| is
+ * as exact as T has it.  A level takes about 6 passes with L = 64, 10 with 8
+ * and 17 with 2 (bisect_kernel 25); one below 1e-5 ||T|| two or three times as
+ * many (a stopping rule of 0.5 eps ||T|| saves 40 of 840 us of chi of Si on 8^3 k
+ * and loses those levels' digits). */
 template <int L>
 __global__ void __launch_bounds__(256) bisect_group_kernel(int N, int nmat, int nb, int mspan, const double *dS,
                                                      const double *eS, const double *gb, double *lamS, double *evals) {
@@ -2575,7 +2576,7 @@ __global__ void __launch_bounds__(256) bisect_group_kernel(int N, int nmat, int 
     const int mat = (int)(g / nb), j = (int)(g % nb);
     const double *d = dl + (mat - m0) * N, *e2 = e2l + (mat - m0) * (N + 1);
     double lo = gb[4 * mat], hi = gb[4 * mat + 1];
-    const double pivmin = gb[4 * mat + 2], tnorm = gb[4 * mat + 3];
+    const double pivmin = gb[4 * mat + 2];
     int clo = 0, chi = N; /* counts below lo and hi (the Gershgorin bounds hold every eigenvalue) */
     double slo = 0.0, shi = 0.0; /* d log|det| at lo and hi; 0 (no step) at the Gershgorin bounds */
     /* 1/q from v_rcp_f64 and one Newton step (a few ulp; the count is that of
@@ -2589,7 +2590,7 @@ __global__ void __launch_bounds__(256) bisect_group_kernel(int N, int nmat, int 
     double x0 = 0.5 * (lo + hi), lam = x0; /* lane 0's probe once the eigenvalue is alone */
     bool alone = false;
     for (int it = 0; it < 160; it++) {
-        const double tol = 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + 4.0 * pivmin + 0.0625 * DBL_EPSILON * tnorm;
+        const double tol = 2.0 * DBL_EPSILON * fmax(fabs(lo), fabs(hi)) + 4.0 * pivmin;
         if (hi - lo <= tol) {
             lam = 0.5 * (lo + hi);
             break;
@@ -2685,7 +2686,7 @@ __global__ void __launch_bounds__(256) bisect_group_kernel(int N, int nmat, int 
             const bool low = fabs(stl) <= fabs(sth);
             const double step = low ? stl : sth, xb = low ? lo : hi;
             const double cand = xb - step;
-            if (fabs(step) <= 2.0 * DBL_EPSILON * fabs(xb) + 4.0 * pivmin + 0.5 * DBL_EPSILON * tnorm && cand >= lo && cand <= hi) {
+            if (fabs(step) <= 2.0 * DBL_EPSILON * fabs(xb) + 4.0 * pivmin && cand >= lo && cand <= hi) {
                 lam = cand;
                 break;
             }

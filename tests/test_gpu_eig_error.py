@@ -79,3 +79,18 @@ def test_register_tiles(monkeypatch, gcut2):
     want = _exact(s, K, 20, 2)
     rms = lambda e: np.sqrt(((e[:, ::2] - want) ** 2).mean())  # noqa: E731
     assert rms(got) < 1.1 * rms(other), (rms(got), rms(other))
+
+
+# one lane per level to 64
+@pytest.mark.parametrize("nk", [1, 300, 3000, 70000])
+def test_small_levels(nk):
+    """Without a potential H is diagonal and so is T, and the lowest level is a |K|^2: down to 1e-19 ||H|| it has to
+    come out to a few roundings of its own (4 for the squares and their sum, 2 for the stopping rule, twice for the ratio)."""
+    inp = capi.Input(["-crystal", "zb", "-a", "5.43", "-vg", "3,4,8,11" + ",0" * 8, "-gcut", repr(12.0 ** 0.5)])
+    ctx = capi.Context(0)
+    ctx.set_system(inp.system(), inp)
+    kap = 2.0 ** np.linspace(-30, -3, nk).round() if nk > 1 else np.array([2.0 ** -30])
+    e = ctx.bands(kap[:, None] * np.array([[1.0, 0.5, 0.25]]), 2, 0.0) / kap[:, None] ** 2
+    top = ctx.bands(np.array([[0.125, 0.0625, 0.03125]]), 2, 0.0)[0, 0] * 64
+    ctx.close()
+    assert np.abs(e / top - 1).max() < 12 * np.finfo(float).eps
