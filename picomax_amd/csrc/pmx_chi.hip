@@ -33,6 +33,7 @@
  * which equals the reference's reO / imO (including its cross-spin terms in
  * reO only) summed per transition.
  */
+#include "pmx_broadening.h"
 #include "pmx_device.h"
 
 #include <algorithm>
@@ -56,7 +57,6 @@ __device__ __forceinline__ zd cconj(zd a) { return zd{a.x, -a.y}; }
 typedef double dx4 __attribute__((ext_vector_type(4)));
 typedef float fx4 __attribute__((ext_vector_type(4)));
 
-constexpr int MAX_NT = 20; /* 4 waves x 5 orders in the MFMA kernel */
 constexpr int TILE = 16;
 
 /* ------------------------------------------------------------------
@@ -2749,138 +2749,10 @@ __global__ void kkmat_bf3_kernel(int nfreq, int NFp, int NFc, double dfreq, __bf
     }
 }
 
-/* host: one row of Taylor coefficients h^n delta^(n)(x)/n!, n < NT */
-void taylor_row(int delta, double eps, double h, double x, int NT, double *row) {
-    if (delta == 1) {
-        /* (1/pi) Im[(-1)^n / (x - i eps)^(n+1)] h^n */
-        std::complex<double> z(x, -eps), inv = 1.0 / z, pw = inv;
-        double hn = 1.0, sg = 1.0;
-        for (int n = 0; n < NT; n++) {
-            row[n] = sg * hn * pw.imag() / PMX_PI;
-            pw *= inv;
-            hn *= h;
-            sg = -sg;
-        }
-    } else {
-        /* a_{n+1} = -(x a_n + a_{n-1}) / (eps^2 (n+1)), a_0 = g(x) */
-        double am1 = 0.0, a0 = std::exp(-0.5 * x * x / (eps * eps)) / (eps * std::sqrt(2.0 * PMX_PI));
-        double hn = 1.0;
-        for (int n = 0; n < NT; n++) {
-            row[n] = hn * a0;
-            double a1 = -(x * a0 + am1) / (eps * eps * (n + 1));
-            am1 = a0;
-            a0 = a1;
-            hn *= h;
-        }
-    }
-}
-
-/* host: the expansion of delta over a bin, economised.  The Taylor series
- * about the bin centre needs NT orders because it spends its accuracy at
- * s = 0; rewritten in Chebyshev polynomials T_n(s) on |s| <= 1 its
- * coefficients fall like (1/r + sqrt(1/r^2 + 1))^-n instead of r^n
- * (Lorentzian, r = (df/2)/epsilon), so M < NT of them leave the same rms
- * error.  The kept part is written back in powers of s, so moments and
- * convolution run as before with M orders in place of NT (Lorentzian r = 0.2:
- * 12 for 16 in FP64, 7 for 9 on the mixed paths; the rank update, the
- * convolution and the moments' memory are all linear in it). */
-struct Economised {
-    int M, NX;             /* orders kept; Taylor orders the coefficients are taken from */
-    std::vector<double> E; /* [M][NX]: Taylor coefficients -> kept powers */
-};
-
-/* NT: the order count of the plain series.  slack: the rms error allowed over
- * that of NT Taylor terms (1 in FP64; 4 on the mixed paths, where both are
- * far below the rounding of 32-bit sums). */
-Economised economise(int delta, double eps, double df, int NT, double slack) {
-    const double r = 0.5 * df / eps, h = 0.5 * df;
-    Economised ec;
-    int NX = NT + 4;
-    for (double t = std::pow(r, NX); t > 1e-16 && NX < 64; t *= r) NX++;
-    /* A[k][n]: the T_k coefficient of s^n; B[n][k]: the s^n coefficient of T_k */
-    std::vector<long double> A((size_t)NX * NX, 0.0L), B((size_t)NX * NX, 0.0L);
-    A[0] = 1.0L;
-    for (int n = 1; n < NX; n++) /* s T_k = (T_{k+1} + T_{|k-1|}) / 2 */
-        for (int k = 0; k < n; k++) {
-            const long double v = A[(size_t)k * NX + n - 1];
-            if (k == 0) A[(size_t)1 * NX + n] += v;
-            else {
-                A[(size_t)(k + 1) * NX + n] += 0.5L * v;
-                A[(size_t)(k - 1) * NX + n] += 0.5L * v;
-            }
-        }
-    B[0] = 1.0L;
-    if (NX > 1) B[(size_t)1 * NX + 1] = 1.0L;
-    for (int k = 2; k < NX; k++)
-        for (int n = 0; n < NX; n++)
-            B[(size_t)n * NX + k] = (n > 0 ? 2.0L * B[(size_t)(n - 1) * NX + k - 1] : 0.0L) - B[(size_t)n * NX + k - 2];
-    /* the offsets near the peak, where both series are at their worst */
-    const int Dm = (int)(4.0 * eps / df) + 1;
-    const int step = std::max(1, Dm / 32);
-    std::vector<double> row(NX), tail(NX + 1, 0.0);
-    double worst = 0.0;
-    for (int D = -1; D <= Dm; D += (D < 8 ? 1 : step)) { /* delta is even: D and -1 - D mirror each other */
-        taylor_row(delta, eps, h, (D + 0.5) * df, NX, row.data());
-        double t2 = 0.0;
-        for (int n = NX - 1; n >= 0; n--) {
-            long double a = 0.0L;
-            for (int m = n; m < NX; m += 2) a += A[(size_t)n * NX + m] * row[m];
-            t2 += 0.5 * (double)(a * a); /* rms over the bin of the terms from n on */
-            tail[n] = std::max(tail[n], t2);
-        }
-        worst = std::max(worst, row[NT] * row[NT] / (2.0 * NT + 1.0)); /* rms of the first Taylor term left out */
-    }
-    ec.NX = NX;
-    ec.M = NT;
-    for (int m = 1; m < NT; m++)
-        if (tail[m] <= slack * slack * worst) {
-            ec.M = m;
-            break;
-        }
-    ec.E.assign((size_t)ec.M * NX, 0.0);
-    for (int n = 0; n < ec.M; n++)
-        for (int m = 0; m < NX; m++) {
-            long double v = 0.0L;
-            for (int k = n; k < ec.M && k <= m; k++) v += B[(size_t)n * NX + k] * A[(size_t)k * NX + m];
-            ec.E[(size_t)n * NX + m] = (double)v;
-        }
-    return ec;
-}
-
-/* host: kernel table K_n(D), n < ec.M, for the W offsets D = f0 - f =
- * Dlo .. Dlo + W - 1 (row D - Dlo) */
-void kernel_table(int delta, double eps, double df, int Dlo, int W, const Economised &ec, std::vector<double> &Kt) {
-    Kt.assign((size_t)W * ec.M, 0.0);
-    std::vector<double> row(ec.NX);
-    for (int Dd = Dlo; Dd < Dlo + W; Dd++) {
-        taylor_row(delta, eps, 0.5 * df, (Dd + 0.5) * df, ec.NX, row.data()); /* x = c_b - w_f */
-        for (int n = 0; n < ec.M; n++) {
-            double v = 0.0;
-            for (int m = ec.NX - 1; m >= n; m--) v += ec.E[(size_t)n * ec.NX + m] * row[m];
-            Kt[(size_t)(Dd - Dlo) * ec.M + n] = v;
-        }
-    }
-}
-
 int window_half(int delta, double eps, double df) {
     int wg = std::max(1, int(6.0 * eps / df));
     int wl = std::max(1, int(50.0 * eps / df));
     return (delta == 1) ? wl : wg;
-}
-
-/* Taylor order for a truncation below tol relative to the peak: with
- * r = (df/2)/epsilon the Lorentzian terms fall like r^n (its poles sit at
- * distance >= epsilon from every expansion point), the Gaussian ones like
- * r^n / sqrt(n!) (Hermite-function bound). */
-int taylor_order(int delta, double eps, double df, double tol) {
-    const double r = 0.5 * df / eps;
-    if (r >= 0.6) return -1;
-    double term = 1.0;
-    for (int n = 1; n <= MAX_NT; n++) {
-        term *= (delta == 0) ? r / std::sqrt((double)n) : r;
-        if (term < tol) return n;
-    }
-    return -1;
 }
 
 template <class T> int upload(hipStream_t s, DBuf<T> &b, const std::vector<T> &h) {
@@ -3170,7 +3042,7 @@ static int chi_run(pmx_ctx *c, const pmx_chi_params *p, double *dRe, double *dIm
                           (p->precision == PMX_PREC_FP64) ? 1e-11 : 1e-6);
         if (NT < 0 || NT > MAX_NT) direct = true;
         else {
-            ec = economise(p->delta, p->epsilon, df, NT, p->precision == PMX_PREC_FP64 ? 1.0 : 4.0);
+            ec = economise(p->delta, p->epsilon, df, NT);
             NT = ec.M;
         }
     }
