@@ -2764,14 +2764,29 @@ template <class T> int upload(hipStream_t s, DBuf<T> &b, const std::vector<T> &h
 
 } // namespace
 
-/* the buffers of the adjoint of chi: kept with the context, grown to the largest
- * call (at most 4 GB of eigenvectors at k and as much at k+q) and freed with it.
+/* the buffers of the adjoint of chi: kept with the context up to 1 GiB together and
+ * freed with it; a call that needs more gives them all back at its end (trim).
  * Allocated and freed by each call they cost 2.2 ms of a fit step of GaAs on 12^3 k
- * (14.2 -> 12.0 ms). */
+ * (14.2 -> 12.0 ms, 0.7 GB). */
 struct AdjWork {
     DBuf<double> Kd, KQd, KWd, evk, evkq, dEd, wtd, gdE, gEk, gEkq, gr, gi, gr0, gi0, KkT, out, gReD, gImD;
     DBuf<zd> vk, vkq, X, gX, gk, gkq, Y, ucd, wAd, wSd, gZ;
     DBuf<int> invd, nc, nv, tbase, pos, bad, act, arow, live;
+    static constexpr size_t KEEP = (size_t)1 << 30;
+    void trim() {
+        DBuf<double> *d[] = {&Kd,  &KQd,  &KWd, &evk, &evkq, &dEd, &wtd, &gdE,  &gEk,
+                             &gEkq, &gr, &gi,  &gr0, &gi0,  &KkT, &out, &gReD, &gImD};
+        DBuf<zd> *z[] = {&vk, &vkq, &X, &gX, &gk, &gkq, &Y, &ucd, &wAd, &wSd, &gZ};
+        DBuf<int> *i[] = {&invd, &nc, &nv, &tbase, &pos, &bad, &act, &arow, &live};
+        size_t bytes = 0;
+        for (auto *b : d) bytes += sizeof(double) * b->n;
+        for (auto *b : z) bytes += sizeof(zd) * b->n;
+        for (auto *b : i) bytes += sizeof(int) * b->n;
+        if (bytes <= KEEP) return;
+        for (auto *b : d) b->release();
+        for (auto *b : z) b->release();
+        for (auto *b : i) b->release();
+    }
 };
 
 struct ChiWork {
@@ -4453,8 +4468,9 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
     const size_t lds_t = sizeof(double) * 4 * (size_t)nch * D;
     if (lds_t > c->lds_max) return set_error(PMX_EINVAL, "NEPS too large for the adjoint");
     /* k-points go in batches of at most 2048 whose two full eigenvector sets
-     * (at k and at k+q, 16 N^2 bytes per k-point each) stay near 4 GB, and so
-     * do the overlaps and their gradients beyond 512: the gradient is a sum
+     * (at k and at k+q, 16 N^2 bytes per k-point each) stay within 4 GB together,
+     * and so do the overlaps and their gradients where a batch has more than 512:
+     * the gradient is a sum
      * over k, so each batch recomputes its eigenpairs and adds its share, and
      * device memory does not grow with the grid.  512 k-points are two matrices
      * per CU, where five of order 89 fit: a fit step of GaAs on 12^3 k takes
@@ -4462,7 +4478,8 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
     size_t kb = std::max<size_t>(16, std::min<size_t>(2048, (size_t)4e9 / (32 * (size_t)N * N + 1)));
     if (kb > 512) {
         const size_t nst = soc ? p->nband : p->nband / 2;
-        kb = std::max<size_t>(512, std::min(kb, (size_t)4e9 / (8 * nst * nst * nch * D + 1))); /* nc nv <= nst^2 / 4 */
+        /* conduction states at k times valence states at k+q: levels may cross the zero between them */
+        kb = std::max<size_t>(512, std::min(kb, (size_t)4e9 / (32 * nst * nst * nch * D + 1)));
     }
     const int KB = (int)std::min<size_t>(kb, nk);
 
@@ -4491,6 +4508,10 @@ extern "C" int pmx_grad_chi(pmx_ctx *c, const pmx_chi_params *p, const double *g
         }
     const size_t nup = (size_t)nel * nq * nfreq;
     if (!c->chi) c->chi = new ChiWork();
+    struct Trim {
+        AdjWork &w;
+        ~Trim() { w.trim(); }
+    } trim{c->chi->adj};
     auto &[Kd, KQd, KWd, evk, evkq, dEd, wtd, gdE, gEk, gEkq, gr, gi, gr0, gi0, KkT, out, gReD, gImD, vk, vkq, X, gX, gk, gkq,
            Y, ucd, wAd, wSd, gZ, invd, nc, nv, tbase, pos, bad, act, arow, live] = c->chi->adj;
     int rc;
