@@ -2693,6 +2693,9 @@ __global__ void __launch_bounds__(1024) epsm_ws_kernel(EpsBlock a, zd *work, zd 
 
 constexpr int EPS_REG_N = 127; /* largest N held in registers (two rows a lane, 8 columns in each of 16 waves) */
 
+/* of one matrix: N^3 / 3 complex multiply-adds */
+double epsm_flops(int N) { return 8.0 / 3.0 * N * N * (double)N; }
+
 /* eps_M and ELF of matrices 0 .. nmat - 1 (q, f); the workspace form runs in
  * launches of as many matrices as its ws_entries hold */
 int launch_epsm(pmx_ctx *c, const EpsBlock &a, int nmat, zd *work, size_t ws_entries, zd *epsM, double *elf) {
@@ -3812,6 +3815,7 @@ extern "C" int pmx_epsinv(pmx_ctx *c, int nq, int neps, int nfreq, const double 
     DBuf<double> re, im, el;
     DBuf<zd> scr, em, inv;
     int rc;
+    const double n3 = (double)neps * neps * neps;
     const size_t ws = epsinv ? (size_t)nmat * neps * 2 * neps
                              : (neps <= EPS_REG_N ? 1 : (size_t)std::min(nmat, 2048) * neps * (neps + 1));
     if ((rc = re.ensure(nblk)) || (rc = im.ensure(nblk)) || (rc = el.ensure(nmat)) || (rc = em.ensure(nmat)) ||
@@ -3821,7 +3825,7 @@ extern "C" int pmx_epsinv(pmx_ctx *c, int nq, int neps, int nfreq, const double 
     PMX_CHECK_HIP(hipMemcpyAsync(re.p, ReX, sizeof(double) * nblk, hipMemcpyHostToDevice, st));
     PMX_CHECK_HIP(hipMemcpyAsync(im.p, ImX, sizeof(double) * nblk, hipMemcpyHostToDevice, st));
     {
-        Prof pf(c, "epsinv", 8.0 * neps * neps * 2.0 * neps * nmat, 0.0);
+        Prof pf(c, "epsinv", epsinv ? 16.0 * n3 * nmat : epsm_flops(neps) * nmat, 0.0);
         if (epsinv)
             hipLaunchKernelGGL(epsinv_kernel, dim3(nmat), dim3(256), 0, st, neps, nfreq, re.p, im.p, scr.p, em.p, el.p,
                                inv.p);
@@ -3917,7 +3921,7 @@ extern "C" int pmx_eps_macro(pmx_ctx *c, int nq, const double *Q, int neps, int 
         }
     if ((rc = upload(st, hd, head))) return rc;
     {
-        Prof pf(c, "epsinv", 2.0 * 8.0 * neps * neps * 2.0 * neps * nmat, 0.0);
+        Prof pf(c, "epsinv", 2.0 * epsm_flops(neps) * nmat, 0.0);
         if ((rc = launch_epsm(c, EpsBlock{neps, nfreq, reL.p, imL.p, nullptr, 0.0, hd.p}, nmat, scr.p, ws, emL.p, el.p)) ||
             (rc = launch_epsm(c, EpsBlock{neps, nfreq, reT.p, imT.p, qgd.p, dfreq, nullptr}, nmat, scr.p, ws, emT.p, el.p)))
             return rc;
