@@ -2510,12 +2510,14 @@ __device__ __forceinline__ double lane_f64(double v, int l) {
  * multipliers of all rows (0 for used ones) and the pivot's index in LDS; after
  * the step's one barrier every wave updates its columns right of k, the pivot
  * row's entry read from its lane.  Rows are not swapped.  The two LDS slots
- * alternate.  Instruction issue bounds it (eight instructions a column and step,
+ * alternate.  Instruction issue bounds it (ten instructions a column and step,
  * four of them lane reads; some 60 more for the step), so it matters that a
  * wave works on whole columns: with the rows split over the waves, each finding
  * the pivot of its own, 1000 matrices of N = 59 took 0.26 ms; with the matrix in
  * LDS 0.24 ms (LDS bandwidth); Gauss-Jordan in global memory 5.6 ms; this
- * 0.10 ms.  The stored block has f innermost, so neighbouring f share
+ * 0.105 ms.  A product is formed before it is subtracted, which rounds an entry once
+ * a step (as two FMAs on the entry 0.10 ms, and up to 1.8 times the error of the
+ * inverse).  The stored block has f innermost, so neighbouring f share
  * lines: each XCD takes a range of f. */
 template <int RB, int NW, int CW>
 __global__ void __launch_bounds__(64 * NW) epsm_reg_kernel(EpsBlock a, zd *epsM, double *elf) {
@@ -2594,8 +2596,8 @@ __global__ void __launch_bounds__(64 * NW) epsm_reg_kernel(EpsBlock a, zd *epsM,
                 const zd p{lane_f64(v.x, pl), lane_f64(v.y, pl)};
 #pragma unroll
                 for (int b = 0; b < RB; b++) {
-                    col[b].x = fma(t[b].y, p.y, fma(-t[b].x, p.x, col[b].x));
-                    col[b].y = fma(-t[b].y, p.x, fma(-t[b].x, p.y, col[b].y));
+                    col[b].x -= fma(-t[b].y, p.y, t[b].x * p.x);
+                    col[b].y -= fma(t[b].y, p.x, t[b].x * p.y);
                 }
             };
             if (wave > o) update(x[i]);
@@ -2678,8 +2680,8 @@ __global__ void __launch_bounds__(1024) epsm_ws_kernel(EpsBlock a, zd *work, zd 
 #pragma unroll
                     for (int u = 0; u < 4; u++) {
                         const zd t = cmul(fr[u], ip);
-                        x[u].x = fma(t.y, p.y, fma(-t.x, p.x, x[u].x));
-                        x[u].y = fma(-t.y, p.x, fma(-t.x, p.y, x[u].y));
+                        x[u].x -= fma(-t.y, p.y, t.x * p.x);
+                        x[u].y -= fma(t.y, p.x, t.x * p.y);
                         if (r[u] >= 0 && c <= N) A[(size_t)r[u] * ld + c] = x[u];
                     }
                 }
