@@ -2798,7 +2798,7 @@ struct ChiWork {
     AdjWork adj;
     DBuf<double> Kd, KQd, KWd, evk, dEd, wtd, Ktd, Kkd, Re0, Im0, ReD, ImD; /* evk, vk: [k; k+q] halves */
     DBuf<double> ws, ss, es, qgn;
-    DBuf<zd> vk, Xd, M1, M2, Z1, Z2, Zp, wAd, ucd, wSd; /* Zp: the direct sum's segments */
+    DBuf<zd> vk, Xd, M1, M2, Z1, Z2, Zp, wAd, ucd, wSd; /* Zp: the direct sum's segments, at most 256 MB */
     DBuf<float2> Xf;
     DBuf<float> Ktf, Kkf;
     DBuf<__bf16> kA, kT; /* split-BF16 KK: A rows [Ih | Il | Rh | Rl][M][NFp], K [KhT | KlT][NFc][NFp] */
@@ -2891,10 +2891,6 @@ __global__ void qnext_kernel(int *qstate) {
     if (threadIdx.x == 0) qstate[0] += 1;
 }
 
-/* Workspace of pmx_epsinv_noalloc: device memory that exists from module load
- * to process end, one copy per GPU, so that entry point calls no allocator.
- * Host code never uses this name as an address (on the host it is a stand-in
- * symbol); it uses the per-device pointer from hipGetSymbolAddress below. */
 /* the eigenpairs of the current q of a batch (slot q % nqb) to the slot that a
  * captured step reads */
 __global__ void __launch_bounds__(256) qslot_kernel(const int *qstate, int nqb, size_t nev, size_t nvk, const double *ev,
@@ -2916,6 +2912,10 @@ int q_batch(const pmx_ctx *c, int nk, int nq, size_t bytes_per_k) {
     return (int)std::max<size_t>(1, std::min<size_t>(nq, n > 1 ? n - 1 : 1));
 }
 
+/* Workspace of pmx_epsinv_noalloc: device memory that exists from module load
+ * to process end, one copy per GPU, so that entry point calls no allocator.
+ * Host code never uses this name as an address (on the host it is a stand-in
+ * symbol); it uses the per-device pointer from hipGetSymbolAddress below. */
 constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)32 << 20;
 static __device__ __align__(256) zd scratch[NOALLOC_SCRATCH_BYTES / sizeof(zd)];
 
@@ -3843,10 +3843,12 @@ extern "C" int pmx_epsinv(pmx_ctx *c, int nq, int neps, int nfreq, const double 
     return PMX_OK;
 }
 
-/* pmx_epsinv on device arrays with no device allocation: the Gauss-Jordan
- * workspace is the file-scope scratch array (NOALLOC_SCRATCH_BYTES per GPU),
- * and the (q, f) matrices run in chunks of as many as fit it.  The kernel
- * writes every workspace entry before reading it, so nothing is cleared. */
+/* pmx_epsinv's eps_M and ELF on device arrays with no device allocation: up to
+ * 127 G the elimination runs in registers; above, its workspace is the
+ * file-scope scratch array (NOALLOC_SCRATCH_BYTES per GPU) and the (q, f)
+ * matrices run in chunks of as many as fit it.  The kernel writes every
+ * workspace entry before reading it, so nothing is cleared.  The limit on neps
+ * is that of [eps | I] in this array. */
 extern "C" int pmx_epsinv_noalloc(pmx_ctx *c, int nq, int neps, int nfreq, const double *dReX, const double *dImX,
                                   double *dEpsM, double *dElf) {
     if (!c || !dReX || !dImX || !dEpsM || !dElf) return set_error(PMX_EINVAL, "null pointer");
