@@ -80,18 +80,14 @@ __device__ __forceinline__ zd cdiv(zd a, zd b) {
 __device__ __forceinline__ double cdiv(double a, double b) { return a / b; }
 
 
-/* acc + a b, acc + conj(a) b and acc - a b as chains of FMAs (four for complex) */
+/* acc + a b and acc + conj(a) b as chains of FMAs (four for complex) */
 __device__ __forceinline__ double mad(double acc, double a, double b) { return fma(a, b, acc); }
 __device__ __forceinline__ double madc(double acc, double a, double b) { return fma(a, b, acc); }
-__device__ __forceinline__ double msub(double acc, double a, double b) { return fma(-a, b, acc); }
 __device__ __forceinline__ zd mad(zd c, zd a, zd b) {
     return zd{fma(-a.y, b.y, fma(a.x, b.x, c.x)), fma(a.y, b.x, fma(a.x, b.y, c.y))};
 }
 __device__ __forceinline__ zd madc(zd c, zd a, zd b) {
     return zd{fma(a.y, b.y, fma(a.x, b.x, c.x)), fma(-a.y, b.x, fma(a.x, b.y, c.y))};
-}
-__device__ __forceinline__ zd msub(zd c, zd a, zd b) {
-    return zd{fma(a.y, b.y, fma(-a.x, b.x, c.x)), fma(-a.y, b.x, fma(-a.x, b.y, c.y))};
 }
 
 /* Sum over a full wave (every lane active) by DPP within rows of 16 and
